@@ -499,10 +499,10 @@ int64_t tv_tree_attention_workspace_bytes(int32_t num_partial_slots, int32_t hea
  *
  * out[q, h, :] = sum_k p_k V[k, h/G, :] / sum_k p_k with p_k = exp(s_k - max s) and
  * s_k = scale * q[q,h,:] . K[k, h/G, :] (+ qq_bias[bias_off[r] + local * T + j] for tree
- * key j); key position pos of request r is visible iff pos <= P + local.  Arithmetic,
- * probabilities and the online softmax are fp32.  No plan or workspace: one wave per
- * (packed row, KV head), reading every metadata value from device memory, so the launch
- * is graph-capturable as is.  Out-of-range pages or slots set TV_STATUS_BAD_PAGE and
+ * key j); key position pos of request r is visible iff pos <= P + local.  Products are exact
+ * with fp32 sums, probabilities and the online softmax fp32.  No plan or workspace: a
+ * workgroup per 32 score rows of a request and KV head, reading every metadata value from
+ * device memory, so the launch is graph-capturable as is.  Out-of-range pages or slots set TV_STATUS_BAD_PAGE and
  * that key is skipped; a row naming a nonexistent request sets TV_STATUS_BAD_REQUEST.
  */
 typedef struct tv_tree_attention_fp32_args {
@@ -541,6 +541,17 @@ typedef struct tv_tree_attention_fp32_args {
 } tv_tree_attention_fp32_args;
 
 int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* args, void* stream);
+/*
+ * The same, with a caller-owned device workspace that lets a batch of few score rows cut its
+ * keys over several workgroups (one launch more, to merge them).  The bytes a batch of these
+ * shapes wants (0: nothing to cut) do not depend on its lengths, and neither does how its keys
+ * are cut, other than on the live ones: a replayed graph computes what an eager call does.
+ * A null workspace is tv_tree_attention_fp32; one that is too small returns TV_ERR_CAPACITY.
+ */
+int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries, int32_t num_requests, int32_t num_q_heads,
+                                               int32_t num_kv_heads, int32_t head_dim);
+int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* args, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
 /* sizeof(tv_tree_attention_fp32_args) as compiled, for binding layout checks. */
 int64_t tv_sizeof_tree_attention_fp32_args(void);
 

@@ -2,25 +2,47 @@
 //
 // The MI355X form of the reference's scalar FP32 kernel (paged_backend.py:116-213) and
 // of its legacy slot-addressed form (paged_backend.py:20-113): the path for batches the
-// MFMA kernel does not take (f32 operands, head sizes other than 128, query groups the
-// MFMA kernel is not built for, page sizes that are not multiples of 32, trees above
-// 1024 nodes, finite qq_bias values).  The reference runs one program per (packed row,
-// query head).  Here a workgroup of four waves owns four consecutive rows of one request
-// and one KV head with its G query heads, so every K/V row it loads serves 4 x G rows.
+// MFMA kernel does not take (f32 operands, head sizes other than 64, 128 and 256, query
+// groups the MFMA kernel is not built for, page sizes that are not multiples of 32, trees
+// above 2048 nodes, finite qq_bias values).  The reference runs one program per (packed
+// row, query head).
 //
-// Per tile of TK keys (64 up to head_dim 128) of the group's visible range:
-//   the first TK threads resolve the keys' slots (page table, prefix slot vector or tree
-//   slot); all threads stage the K and V rows into LDS as float (coalesced loads, rows
-//   padded to an odd pitch);
-//   each wave, for its own row: lane k scores key k against the row's G query vectors
-//   (LDS broadcast reads), adds the tree key's bias, runs each head's online softmax as
-//   wave reductions (max, then sum) in fp32, and for P.V the lanes own head dimensions
-//   (lane + 64 j) and walk the tile's keys.
-// Accumulators: G_pass x DJ floats per lane with DJ = ceil(D / 64) and G_pass the smallest
-// power of two >= G up to min(16, 64 / DJ); query heads beyond G_pass take further passes
-// over the keys.
+// Work split.  The T x G score rows of one request and KV head (row = node * G + query
+// head) are cut into blocks of 32.  A workgroup of four waves owns one block and a range of
+// the block's visible keys; its waves take the range's 32-key tiles in turn, each with its
+// own online softmax, and meet once at the end (LDS).  A wave therefore needs no barrier
+// and no staging of K/V: it loads its tiles straight into the operand registers of the
+// matrix instructions, and the row blocks of one request find the K/V in L2.  Batches with
+// few blocks cut the keys over up to kMaxSplits workgroups per block, whose partial rows a
+// second kernel merges.  The cut depends on the live lengths and on the launch's shapes
+// only, so a replayed graph computes what an eager launch computes.
+//
+// Products (per 32-key tile and 32-row block, written transposed so that every per-row
+// quantity sits in the two lanes c, c + 32 of row c):
+//   S^T[32 keys x 32 rows] = K . Q^T        A: lane (c, g) holds key c, B: score row c
+//   O^T[dims x 32 rows]   += V^T . P^T      A: lane (c, g) holds dims 64j + 2c, 2c + 1
+//   f32 operands: v_mfma_f32_32x32x2_f32, exact fp32 products with fp32 sums.  Contraction
+//     slot g of step (j, i) of K.Q^T is dim 8j + 4g + i (16-byte loads of both); slot g of
+//     step v of V^T.P^T is the key that S^T register v of half g holds, so the
+//     probabilities feed the product from the registers the scores were computed in.
+//   16-bit operands: v_mfma_f32_32x32x16; the fp32 probability is split into three terms of
+//     the operand type (its rounding, the rounding of the remainder, and that of the rest:
+//     24 bits in bf16, 33 in f16), one product each, so it enters the sum with at least
+//     fp32's precision.
+//
+// What bounds it.  f32: the matrix core, 8192 cycles a tile and wave (a wave's tile takes 10.7 us
+// with two waves a SIMD, 7 us at the core's rate), and the uneven lengths of the workgroups.
+// 16 bits: the loads and the softmax's vector work (3 us a tile) and the workgroup's fixed time
+// (lookups 3, Q and first tile 3, waves' merge 3, partial rows 2.5 us).  Measured, before (a wave
+// per packed row, fp32 vector products, K/V staged in LDS) -> now: 8 f32 requests of 310-3304
+// keys and 18-64 nodes, 32/8 heads x 128: 525 -> 151 us (5.9 GFLOP; 42 us at the f32 matrix
+// rate); 4 bf16 requests of 1204-1998 keys, 24/8 heads x 96, 16-token pages: 481 -> 37 us;
+// 2 x 1500-row bf16 chunks, 32/8 x 128: 7.1 -> 0.69 ms; head size 512, bf16: 7.2 -> 0.87 ms.
 #include <math.h>
 #include <stdint.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "tv_internal.h"
 
@@ -56,7 +78,16 @@ struct Fp32Params {
     int32_t groups;       // query heads per KV head
     int32_t head_dim;
     int32_t block_size;
-    float scale;
+    float scale;          // softmax scale * log2(e): scores are kept in log2 units
+    int32_t splits;       // chunks a row block's keys may be cut into (grid y)
+    int32_t slots;        // workgroups the chip runs at a time
+    int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
+    int32_t kv_heads;
+    int32_t vec;          // K/V rows take vector loads
+    int32_t q_vec;        // Q rows do
+    int64_t unit0;        // first (row block, KV head) of this launch
+    float* ws_o;          // partial rows [row group, KV head, split, 32, head_dim] (splits > 1)
+    float2* ws_ml;        // their (maximum, sum) [row group, KV head, split, 32]
     int32_t* status;
 };
 
@@ -65,17 +96,6 @@ constexpr int kWave = 64;
 __device__ __forceinline__ float to_float(float x) { return x; }
 __device__ __forceinline__ float to_float(__bf16 x) { return static_cast<float>(x); }
 __device__ __forceinline__ float to_float(_Float16 x) { return static_cast<float>(x); }
-
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-    return x;
-}
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-    return x;
-}
 
 __device__ __forceinline__ void store_value(const Fp32Params& p, int64_t index, float x) {
     if (p.out_dtype == TV_F32) {
@@ -87,26 +107,35 @@ __device__ __forceinline__ void store_value(const Fp32Params& p, int64_t index, 
     }
 }
 
-constexpr int kRowsPerGroup = 4;    // waves per workgroup: consecutive rows of one request
-constexpr int kThreadsFp32 = kWave * kRowsPerGroup;
+constexpr int kBlockRows = 32;      // score rows of a workgroup
+constexpr int kTile = 32;           // keys of a tile
+constexpr int kWaves = 4;           // waves of a workgroup: they take its tiles in turn
+constexpr int kThreadsFp32 = kWave * kWaves;
+constexpr int kMaxSplits = 16;
+constexpr int kCus = 256;           // compute units of an MI355X
+constexpr int64_t kCutRows = 4096;  // partial row blocks a workspace holds at most
+// Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
+// rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
+constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
+constexpr float kLog2eF = 1.4426950408889634f;
 
-// The launch numbers the row groups of request r from start(r) = cu[r] / 4 + r on: the
-// ranges are disjoint and increasing (start(r + 1) - start(r) >= ceil(T_r / 4)), so a grid
-// of Q / 4 + R + 1 workgroups covers every group with at most one idle workgroup per
-// request, and consecutive workgroups (spread over the XCDs) all have work.
-__device__ __forceinline__ int64_t group_start(const int32_t* cu, int r) {
-    return static_cast<int64_t>(cu[r] / kRowsPerGroup) + r;
+// The launch numbers the row blocks of request r from start(r) = floor(cu[r] * G / 32) + r on:
+// the ranges are disjoint and increasing (start(r + 1) - start(r) >= ceil(T_r * G / 32)), so a
+// grid of floor(Q * G / 32) + R + 1 numbers covers every block with at most one idle number per
+// request, whatever the (live) node counts.
+__device__ __forceinline__ int64_t group_start(const int32_t* cu, int groups, int r) {
+    return static_cast<int64_t>(cu[r]) * groups / kBlockRows + r;
 }
 
 // The request whose group range holds workgroup b: the last r with start(r) <= b, by a
 // 64-way search of the wave (two rounds of loads up to 4096 requests).
-__device__ int request_of_group(const int32_t* cu, int num_requests, int64_t b) {
+__device__ int request_of_group(const int32_t* cu, int groups, int num_requests, int64_t b) {
     const int lane = threadIdx.x & (kWave - 1);
     int lo = 0, hi = num_requests;   // start(lo) <= b; the answer is in [lo, hi)
     while (hi - lo > 1) {
         const int step = (hi - lo + kWave - 1) / kWave;
         const int r = lo + lane * step;
-        const bool le = r < hi && group_start(cu, r) <= b;
+        const bool le = r < hi && group_start(cu, groups, r) <= b;
         const uint64_t mask = __ballot(le);   // lanes 0 .. k set: start() increases with r
         const int last = 63 - __builtin_clzll(mask | 1ull);
         lo += last * step;
@@ -115,285 +144,802 @@ __device__ int request_of_group(const int32_t* cu, int num_requests, int64_t b) 
     return lo;
 }
 
-// Keys per LDS tile: 64 up to head_dim 128, fewer above (the K and V tiles stay near 66 KiB).
-template <int DJ>
-struct TileShape {
-    static constexpr int TK = DJ <= 2 ? 64 : 64 * 2 / DJ;
-    static constexpr int PITCH = kWave * DJ;          // LDS row of one query head (floats)
-    // K/V rows padded by 4 floats: 16-byte aligned, and a lane-per-key 16-byte read of 16
-    // lanes covers the 64 banks once.
-    static constexpr int KV_PITCH = kWave * DJ + 4;
-    static constexpr int KPW = TK / kRowsPerGroup;    // keys each wave stages per tile
+// One workgroup's work: a row block of a request, and the block's chunk of the visible keys.
+struct RowBlock {
+    int r, row0, rows, nodes, prefix;   // rows: score rows of the block (<= 32)
+    int64_t tree0;                      // the request's first packed row
+    int64_t number;                     // the block's number (group_start), which places its partial rows
+    int tiles;                          // 32-key tiles any row of the block can see
+    int seq;                            // ... keys
+    int chunk, part;                    // tiles of a chunk, this workgroup's chunk
 };
 
-// A score more than this far above a row's reference maximum (natural-log units) raises
-// the maximum; below it probabilities stay <= e^8, which fp32 holds with its full
-// relative precision, so the result is the same online softmax with rare rescales.
-constexpr float kRaiseMargin = 8.f;
-
-// T: operand type; DJ: head dimensions per lane (D <= 64 * DJ); GP: query heads per pass
-// (the launch picks the smallest power of two >= G, at most 16 and at most 64 / DJ, so
-// G_pass x DJ accumulators fit).  Workgroup: rows local0 .. local0 + 3 of one request and
-// one KV head.  Software pipeline over tiles of TK keys: while tile t is computed, the K/V
-// loads of tile t + 1 (slots resolved one iteration earlier) and the slot lookups of
-// tile t + 2 are in flight; tile t's K/V rows, staged in LDS as float, serve all four
-// rows.  Each wave runs its own row: lane k scores key k against the row's G query
-// vectors, the row's reference maximum is raised only when a score exceeds it by
-// kRaiseMargin (a ballot; the wave reduction runs then), probabilities and per-lane sums
-// use it, and for P.V the lanes own head dimensions.
-template <typename T, int DJ, int GP>
-__global__ void __launch_bounds__(kThreadsFp32)
-tree_attention_fp32_kernel(const Fp32Params p) {
-    typedef TileShape<DJ> S;
-    constexpr int TK = S::TK, PITCH = S::PITCH, KV_PITCH = S::KV_PITCH, KPW = S::KPW;
-    static_assert(GP * DJ <= 64, "accumulators per lane");
-    static_assert(TK <= kThreadsFp32 && TK % 4 == 0, "one slot lookup per thread, 4-key P.V steps");
-    __shared__ __attribute__((aligned(16))) float q_lds[kRowsPerGroup][GP * PITCH];
-    __shared__ __attribute__((aligned(16))) float p_lds[kRowsPerGroup][GP * TK];
-    __shared__ __attribute__((aligned(16))) float k_lds[TK * KV_PITCH];
-    __shared__ __attribute__((aligned(16))) float v_lds[TK * KV_PITCH];
-    __shared__ int64_t kbase_lds[2][TK], vbase_lds[2][TK];   // element offsets of the rows, -1: missing
-
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int kvh = blockIdx.y;
-    const int r = __builtin_amdgcn_readfirstlane(request_of_group(p.cu, p.num_requests, blockIdx.x));
-    const int local0 = static_cast<int>(blockIdx.x - group_start(p.cu, r)) * kRowsPerGroup;
-    const int P = p.plen[r], nodes = p.cnt[r];
-    if (local0 >= nodes) return;   // the gap after request r's groups
-    if (P < 0) {
-        if (tid == 0) set_status(p.status, TV_STATUS_BAD_REQUEST);
-        return;
+// Fills the block `index` of request r, whose live metadata are given; false for an index past
+// the request's rows and for a request whose live lengths are malformed.
+__device__ __forceinline__ bool block_of_request(const Fp32Params& p, int r, int index, int cu, int nodes, int prefix,
+                                                 RowBlock& b, bool report) {
+    b.r = r;
+    b.row0 = index * kBlockRows;
+    b.prefix = prefix;
+    b.nodes = nodes;
+    b.tree0 = cu;
+    b.number = static_cast<int64_t>(cu) * p.groups / kBlockRows + r + index;
+    const int64_t rows = static_cast<int64_t>(nodes) * p.groups;
+    if (b.row0 >= rows) return false;
+    const int last = static_cast<int>((min(static_cast<int64_t>(b.row0) + kBlockRows, rows) - 1) / p.groups);
+    if (prefix < 0 || cu < 0 || b.tree0 + last >= p.total_queries) {
+        if (report && threadIdx.x == 0) set_status(p.status, TV_STATUS_BAD_REQUEST);
+        return false;
     }
-    const int64_t leader = static_cast<int64_t>(p.cu[r]) + local0;
-    const int rows = min(kRowsPerGroup, nodes - local0);
-    if (leader < 0 || leader + rows > p.total_queries) {
-        if (tid == 0) set_status(p.status, TV_STATUS_BAD_REQUEST);
-        return;
-    }
-    // This wave's row; the metadata must place a request's rows consecutively.
-    const int64_t row = leader + wave;
-    const int local = local0 + wave;
-    bool row_ok = wave < rows;
-    if (row_ok && (p.q2r[row] != r || p.local[row] != local)) {
-        if (lane == 0) set_status(p.status, TV_STATUS_BAD_REQUEST);
-        row_ok = false;
-    }
-    const int D = p.head_dim, B = p.block_size, G = p.groups;
-    const int64_t tree0 = p.cu[r];
-    const int64_t bias_row = p.bias_off[r] + static_cast<int64_t>(local) * nodes;
-    const int seq = P + local0 + rows;    // keys any row of the group can see
-    const int ntiles = (seq + TK - 1) / TK;
-    const int my_end = P + local + 1;     // this row's visible range
-    const int64_t pool_slots = p.num_blocks * B;
-    const T* q = static_cast<const T*>(p.q);
-    const T* k = static_cast<const T*>(p.k);
-    const T* v = static_cast<const T*>(p.v);
-
-    // Slot of key t0 + tid (threads < TK): the load, then the row offsets.
-    auto slot_load = [&](int t0) -> int64_t {
-        const int pos = t0 + tid;
-        if (tid >= TK || pos >= seq) return -1;
-        if (pos >= P) return p.tree_slots[tree0 + (pos - P)];
-        if (p.pslots) {
-            const int64_t at = static_cast<int64_t>(r) * p.ps_s0 + pos;
-            return p.ps_i64 ? static_cast<const int64_t*>(p.pslots)[at]
-                            : static_cast<int64_t>(static_cast<const int32_t*>(p.pslots)[at]);
-        }
-        const int64_t page = p.tables[static_cast<int64_t>(r) * p.t_s0 + pos / B];
-        return (page >= 0 && page < p.num_blocks) ? page * B + pos % B : -2;
-    };
-    auto slot_store = [&](int t0, int64_t slot, int buf) {
-        const int pos = t0 + tid;
-        if (tid >= TK) return;
-        int64_t kb = -1, vb = -1;
-        if (pos < seq) {
-            if (slot < 0 || slot >= pool_slots) {
-                set_status(p.status, TV_STATUS_BAD_PAGE);
-            } else {
-                const int64_t blk = slot / B, off = slot - blk * B;
-                kb = blk * p.k_s0 + off * p.k_s1 + static_cast<int64_t>(kvh) * p.k_s2;
-                vb = blk * p.v_s0 + off * p.v_s1 + static_cast<int64_t>(kvh) * p.v_s2;
-            }
-        }
-        kbase_lds[buf][tid] = kb;
-        vbase_lds[buf][tid] = vb;
-    };
-    // This thread's share of a tile's K and V: wave w stages keys w, w + 4, ..., its lanes
-    // along the head dimension (coalesced); every load is issued before any is used.
-    float kx[KPW][DJ], vx[KPW][DJ];
-    auto kv_load = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < KPW; ++i) {
-            const int key = wave + kRowsPerGroup * i;
-            const int64_t kb = kbase_lds[buf][key], vb = vbase_lds[buf][key];
-#pragma unroll
-            for (int j = 0; j < DJ; ++j) {
-                const int d = lane + kWave * j;
-                const bool ok = kb >= 0 && d < D;
-                kx[i][j] = ok ? to_float(k[kb + d * p.k_s3]) : 0.f;
-                vx[i][j] = ok ? to_float(v[vb + d * p.v_s3]) : 0.f;
-            }
-        }
-    };
-    auto kv_store = [&]() {
-#pragma unroll
-        for (int i = 0; i < KPW; ++i) {
-            const int key = wave + kRowsPerGroup * i;
-#pragma unroll
-            for (int j = 0; j < DJ; ++j) {
-                const int d = lane + kWave * j;
-                k_lds[key * KV_PITCH + d] = kx[i][j];
-                v_lds[key * KV_PITCH + d] = vx[i][j];
-            }
-        }
-    };
-
-    for (int g0 = 0; g0 < G; g0 += GP) {
-        const int gn = min(GP, G - g0);
-        const int head0 = kvh * G + g0;
-        for (int i = lane; i < GP * PITCH; i += kWave) {
-            const int g = i / PITCH, d = i - g * PITCH;
-            float x = 0.f;
-            if (row_ok && g < gn && d < D) x = to_float(q[row * p.q_s0 + static_cast<int64_t>(head0 + g) * p.q_s1 + d]);
-            q_lds[wave][i] = x;
-        }
-        float m[GP], l[GP], acc[GP][DJ];
-#pragma unroll
-        for (int g = 0; g < GP; ++g) {
-            m[g] = -INFINITY;
-            l[g] = 0.f;
-#pragma unroll
-            for (int j = 0; j < DJ; ++j) acc[g][j] = 0.f;
-        }
-        // Pipeline prologue: slots of tiles 0 and 1, K/V loads of tile 0.
-        __syncthreads();   // the previous pass's LDS reads are done
-        slot_store(0, slot_load(0), 0);
-        __syncthreads();
-        kv_load(0);
-        if (ntiles > 1) slot_store(TK, slot_load(TK), 1);
-        int64_t next_slot = -1;   // slot of key (t + 1) * TK + tid, loaded during iteration t - 1
-        for (int t = 0; t < ntiles; ++t) {
-            const int t0 = t * TK;
-            __syncthreads();   // every wave is done with tile t - 1 (its K/V rows and its slot buffer)
-            // Tile t + 1's slots go into the buffer tile t - 1 used: only after the barrier, since
-            // every wave reads its tile's slot buffer in its own compute (the visibility test).
-            if (t >= 1 && t + 1 < ntiles) slot_store(t0 + TK, next_slot, (t + 1) & 1);
-            kv_store();
-            __syncthreads();   // tile t is staged; tile t + 1's slots are in LDS
-            if (t + 1 < ntiles) kv_load((t + 1) & 1);
-            next_slot = t + 2 < ntiles ? slot_load(t0 + 2 * TK) : -1;
-            if (row_ok) {
-                const int pos = t0 + lane;
-                bool visible = lane < TK && pos < my_end && kbase_lds[t & 1][lane < TK ? lane : 0] >= 0;
-                float bias = 0.f;
-                if (visible && pos >= P) {
-                    bias = p.bias[bias_row + (pos - P)];
-                    if (bias == -INFINITY) visible = false;
-                }
-                float sc[GP];
-#pragma unroll
-                for (int g = 0; g < GP; ++g) sc[g] = 0.f;
-                if (visible) {
-                    const float* kr = k_lds + (lane < TK ? lane : 0) * KV_PITCH;
-#pragma unroll 2
-                    for (int d = 0; d < D; d += 4) {
-                        const float4 kv4 = *reinterpret_cast<const float4*>(kr + d);
-#pragma unroll
-                        for (int g = 0; g < GP; ++g) {
-                            const float4 qv = *reinterpret_cast<const float4*>(&q_lds[wave][g * PITCH + d]);
-                            sc[g] = fmaf(qv.x, kv4.x, sc[g]);
-                            sc[g] = fmaf(qv.y, kv4.y, sc[g]);
-                            sc[g] = fmaf(qv.z, kv4.z, sc[g]);
-                            sc[g] = fmaf(qv.w, kv4.w, sc[g]);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int g = 0; g < GP; ++g) {
-                    const float score = visible ? fmaf(sc[g], p.scale, bias) : -INFINITY;
-                    if (__ballot(score > m[g] + kRaiseMargin)) {   // rare after the first tile
-                        const float m_new = fmaxf(m[g], wave_max(score));
-                        const float alpha = expf(m[g] - m_new);   // 0 while m[g] is -inf
-                        l[g] *= alpha;
-#pragma unroll
-                        for (int j = 0; j < DJ; ++j) acc[g][j] *= alpha;
-                        m[g] = m_new;
-                    }
-                    const float pr = score == -INFINITY ? 0.f : expf(score - m[g]);
-                    l[g] += pr;
-                    if (lane < TK) p_lds[wave][g * TK + lane] = pr;
-                }
-                // P.V over the tile's keys (the wave reads only its own probabilities).
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                const int keys = min(TK, my_end - t0);
-                for (int kk = 0; kk < keys; kk += 4) {
-                    float vv[4][DJ];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-#pragma unroll
-                        for (int j = 0; j < DJ; ++j) vv[u][j] = v_lds[(kk + u) * KV_PITCH + lane + kWave * j];
-                    }
-#pragma unroll
-                    for (int g = 0; g < GP; ++g) {
-                        const float4 pg = *reinterpret_cast<const float4*>(&p_lds[wave][g * TK + kk]);
-#pragma unroll
-                        for (int j = 0; j < DJ; ++j) {
-                            acc[g][j] = fmaf(pg.x, vv[0][j], acc[g][j]);
-                            acc[g][j] = fmaf(pg.y, vv[1][j], acc[g][j]);
-                            acc[g][j] = fmaf(pg.z, vv[2][j], acc[g][j]);
-                            acc[g][j] = fmaf(pg.w, vv[3][j], acc[g][j]);
-                        }
-                    }
-                }
-            }
-        }
-        if (row_ok) {
-#pragma unroll
-            for (int g = 0; g < GP; ++g) {
-                const float inv = 1.f / wave_sum(l[g]);
-                const int64_t base = row * p.o_s0 + static_cast<int64_t>(head0 + g) * p.o_s1;
-#pragma unroll
-                for (int j = 0; j < DJ; ++j) {
-                    const int d = lane + kWave * j;
-                    if (g < gn && d < D) store_value(p, base + d, acc[g][j] * inv);
-                }
-            }
-        }
-    }
+    b.rows = static_cast<int>(min(static_cast<int64_t>(kBlockRows), rows - b.row0));
+    b.seq = prefix + last + 1;
+    b.tiles = (b.seq + kTile - 1) / kTile;
+    b.chunk = b.tiles;
+    b.part = 0;
+    return true;
 }
 
-template <typename T, int DJ>
-void launch_for_dims(const Fp32Params& p, const dim3& grid, hipStream_t s) {
-    constexpr int kMaxPass = 64 / DJ < 16 ? 64 / DJ : 16;
-    int gp = 2;
-    while (gp < p.groups && gp < kMaxPass) gp *= 2;
-    switch (gp) {
-        case 2: hipLaunchKernelGGL((tree_attention_fp32_kernel<T, DJ, 2>), grid, dim3(kThreadsFp32), 0, s, p); break;
-        case 4: hipLaunchKernelGGL((tree_attention_fp32_kernel<T, DJ, 4>), grid, dim3(kThreadsFp32), 0, s, p); break;
-        case 8: hipLaunchKernelGGL((tree_attention_fp32_kernel<T, DJ, 8>), grid, dim3(kThreadsFp32), 0, s, p); break;
-        default:
-            hipLaunchKernelGGL((tree_attention_fp32_kernel<T, DJ, kMaxPass>), grid, dim3(kThreadsFp32), 0, s, p);
-            break;
+// Wave-wide sums and maxima in every lane, with DPP moves (shifts within rows of 16 lanes, then
+// row broadcasts: lane 63 ends with the whole); a lane without a source reads 0.
+template <int kCtrl, int kRowMask = 0xf>
+__device__ __forceinline__ int dpp(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, kCtrl, kRowMask, 0xf, false);
+}
+__device__ __forceinline__ int prefix_sum(int x) {   // inclusive
+    x += dpp<0x111>(x);
+    x += dpp<0x112>(x);
+    x += dpp<0x114>(x);
+    x += dpp<0x118>(x);
+    x += dpp<0x142, 0xa>(x);
+    x += dpp<0x143, 0xc>(x);
+    return x;
+}
+__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(prefix_sum(x), kWave - 1); }
+__device__ __forceinline__ float wave_total(float x) {
+    auto move = [](float v, auto f) { return __builtin_bit_cast(float, f(__builtin_bit_cast(int, v))); };
+    x += move(x, dpp<0x111>);
+    x += move(x, dpp<0x112>);
+    x += move(x, dpp<0x114>);
+    x += move(x, dpp<0x118>);
+    x += move(x, dpp<0x142, 0xa>);
+    x += move(x, dpp<0x143, 0xc>);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), kWave - 1));
+}
+__device__ __forceinline__ int wave_max(int x) {   // of non-negative values
+    x = max(x, dpp<0x111>(x));
+    x = max(x, dpp<0x112>(x));
+    x = max(x, dpp<0x114>(x));
+    x = max(x, dpp<0x118>(x));
+    x = max(x, dpp<0x142, 0xa>(x));
+    x = max(x, dpp<0x143, 0xc>(x));
+    return __builtin_amdgcn_readlane(x, kWave - 1);
+}
+
+// The cut of a batch whose keys are split (p.splits > 1, at most kCutRequests requests), the
+// same in every wave that computes it: chunks of at most `target` tiles, so that the workgroups
+// fill the chip once (p.slots of them run at a time: a part-filled second round would double the
+// launch), or as many times as the row blocks alone do.  Lane l holds request l.
+constexpr int kCutRequests = kWave;
+struct Cut {
+    int cu, nodes, prefix;   // the request's live metadata
+    int blocks, tiles;       // its row blocks and the tiles of its keys
+    int target;
+};
+
+__device__ __forceinline__ int chunks_of(int tiles, int target) {
+    return static_cast<int>((static_cast<uint32_t>(tiles) + target - 1) / static_cast<uint32_t>(target));
+}
+// Tiles of one of `parts` even chunks, in whole turns of the waves.
+__device__ __forceinline__ int chunk_tiles(int tiles, int parts) {
+    return ((tiles + parts - 1) / parts + kWaves - 1) / kWaves * kWaves;
+}
+
+__device__ __forceinline__ Cut plan_cut(const Fp32Params& p) {
+    Cut cut = {0, 0, 0, 0, 0, 1};
+    const int r = threadIdx.x & (kWave - 1);
+    if (r < p.num_requests) {
+        cut.cu = p.cu[r];
+        cut.nodes = p.cnt[r];
+        cut.prefix = p.plen[r];
+        if (cut.nodes > 0 && cut.prefix >= 0 && cut.nodes <= p.total_queries) {
+            cut.blocks = static_cast<int>((static_cast<int64_t>(cut.nodes) * p.groups + kBlockRows - 1) / kBlockRows);
+            cut.tiles = static_cast<int>((static_cast<int64_t>(cut.prefix) + cut.nodes + kTile - 1) / kTile);
+        } else if (blockIdx.x == 0 && cut.nodes != 0) {
+            set_status(p.status, TV_STATUS_BAD_REQUEST);
+        }
     }
+    const int units = wave_total(cut.blocks) * p.kv_heads;
+    const int longest = wave_max(cut.tiles);
+    const int slots = p.slots * max(1, (units + p.slots - 1) / p.slots);
+    const float work = wave_total(static_cast<float>(cut.blocks) * static_cast<float>(cut.tiles)) * p.kv_heads;
+    const int even = static_cast<int>(fminf(work / slots, 1e9f));
+    int target = max(max(even, p.min_chunk), (longest + p.splits - 1) / p.splits);
+    target = (target + kWaves - 1) / kWaves * kWaves;
+    // Last chunks are short, so the even share makes a few workgroups too many: longer chunks
+    // until they fit (each step is an eighth; 16 of them are an uncut batch's length).
+    for (int i = 0; i < 16 && target < longest; ++i) {
+        if (wave_total(cut.blocks * chunks_of(cut.tiles, target)) * p.kv_heads <= slots) break;
+        target += max(kWaves, target / 8 / kWaves * kWaves);
+    }
+    cut.target = target;
+    return cut;
+}
+
+// The block and chunk of index u (blocks and chunks of request 0 first, chunk fastest); false
+// past the last.
+__device__ __forceinline__ bool cut_block(const Fp32Params& p, const Cut& cut, int u, RowBlock& b, bool& live) {
+    const int parts = chunks_of(cut.tiles, cut.target);
+    const int mine = cut.blocks * parts, sum = prefix_sum(mine);
+    const uint64_t past = __ballot(sum > u);
+    if (!past) return false;
+    const int l = __builtin_ctzll(past);
+    const int np = __builtin_amdgcn_readlane(parts, l);
+    const int index = u - __builtin_amdgcn_readlane(sum - mine, l), block = index / np;
+    live = block_of_request(p, l, block, __builtin_amdgcn_readlane(cut.cu, l), __builtin_amdgcn_readlane(cut.nodes, l),
+                            __builtin_amdgcn_readlane(cut.prefix, l), b, true);
+    if (live) {
+        b.chunk = chunk_tiles(__builtin_amdgcn_readlane(cut.tiles, l), np);
+        b.part = index - block * np;
+        live = b.part * b.chunk < b.tiles;   // an early block sees fewer keys than its request holds
+    }
+    return true;
+}
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+// The same value, computed where it is used: keeps the many addresses of a rare or strided path
+// from being held in registers across the tile loop.
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
 
 template <typename T>
-void launch_for_type(const Fp32Params& p, int32_t kv_heads, hipStream_t s) {
-    // One workgroup per group of four rows of a request (group_start); the grid depends
-    // only on the packed row and request counts, which a captured graph keeps fixed.
-    const int64_t groups = static_cast<int64_t>(p.total_queries) / kRowsPerGroup + p.num_requests + 1;
-    const dim3 grid(static_cast<uint32_t>(groups), static_cast<uint32_t>(kv_heads));
-    if (p.head_dim <= 64) {
-        launch_for_dims<T, 1>(p, grid, s);
-    } else if (p.head_dim <= 128) {
-        launch_for_dims<T, 2>(p, grid, s);
-    } else if (p.head_dim <= 256) {
-        launch_for_dims<T, 4>(p, grid, s);
+struct Op;
+template <>
+struct Op<__bf16> {
+    typedef bf16x8_t vec;
+    static __device__ __forceinline__ f32x16 mfma(vec a, vec b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+    }
+    // log2 of the factor the probabilities carry (it cancels against the row sum).
+    static constexpr float kShift = 0.f;
+};
+template <>
+struct Op<_Float16> {
+    typedef f16x8_t vec;
+    static __device__ __forceinline__ f32x16 mfma(vec a, vec b, f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+    }
+    // Probabilities up to 2^8 become at most 2^15: the three f16 terms of one then reach down
+    // to 2^-31 of a probability of 1 instead of f16's 2^-24.
+    static constexpr float kShift = 7.f;
+};
+template <>
+struct Op<float> {
+    static constexpr float kShift = 0.f;
+};
+
+// A score more than this far above a row's reference maximum (log2 units) raises the
+// maximum; below it probabilities stay <= 2^8, which fp32 holds with its full relative
+// precision, so the result is the same online softmax with rare rescales.
+constexpr float kRaiseMargin = 8.f;
+
+// T: operand type; DIM: the head size, or (EXACT false) an upper bound of it in {64, 128, 256,
+// 512} with loads and products past p.head_dim left out, and element loads where the rows do not
+// take vector ones.
+template <typename T, int DIM, bool EXACT>
+__device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock& b, const int kvh) {
+    constexpr bool F32 = sizeof(T) == 4;
+    constexpr int DP = (DIM + 63) / 64 * 64;               // padded head size
+    constexpr int NB = DP / 32;                            // 32-dim output blocks
+    constexpr int SLAB = DP == 128 ? 128 : 64;             // dims of K and V held in registers at a time
+    constexpr int SLABS = DP / SLAB;
+    constexpr int KSTEP = F32 ? 8 : 16;                    // dims of a 16-byte K load of both lane halves
+    constexpr int KV4 = SLAB / KSTEP;                      // K loads per lane and slab
+    constexpr int SB = SLAB / 64;                          // 64-dim output pairs per slab
+    constexpr int QPITCH = F32 ? DP + 4 : DP / 2 + 4;      // LDS row of Q in 4-byte words: 16-byte reads conflict free
+    constexpr int OPITCH = DP + 2;                         // LDS row of O: 8-byte accesses conflict free
+    constexpr int Q_WORDS = kBlockRows * QPITCH, O_WORDS = kBlockRows * OPITCH;
+    __shared__ __attribute__((aligned(16))) uint32_t smem[Q_WORDS > 2 * O_WORDS ? Q_WORDS : 2 * O_WORDS];
+    __shared__ uint64_t rows_lds[kWaves][2][2][kTile];     // addresses of the tile's K and V rows
+    __shared__ float2 ml_lds[kWaves][kBlockRows];
+
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), c = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int D = EXACT ? DIM : p.head_dim;
+    const int B = p.block_size, G = p.groups;
+    const int tbeg = b.part * b.chunk, tend = min(b.tiles, tbeg + b.chunk);
+
+    // This lane's score row.  Its metadata, the first tile's slots and the Q rows are loaded before
+    // any of them is used: one round trip instead of four.
+    const int row = b.row0 + c;
+    const int local = row / G;
+    const int64_t packed = b.tree0 + local;
+    const int P = b.prefix;
+    const bool in_block = c < b.rows;
+    const int row_request = in_block ? p.q2r[packed] : b.r, row_local = in_block ? p.local[packed] : local;
+    const int64_t bias_base = p.bias_off[b.r];
+    const int64_t pool_slots = p.num_blocks * B;
+    const float cs = p.scale;
+
+    // Slot of key t0 + c of a tile.  Lanes of half 0 follow the key's K row, those of half 1 its V row.
+    const bool pow2 = (B & (B - 1)) == 0;
+    const int bshift = __builtin_ctz(B);
+    auto slot_load = [&](int t0) __attribute__((always_inline)) -> int64_t {
+        const int pos = t0 + c;
+        if (pos >= b.seq) return -1;
+        if (pos >= P) return p.tree_slots[b.tree0 + (pos - P)];
+        if (p.pslots) {
+            const int64_t at = static_cast<int64_t>(b.r) * p.ps_s0 + pos;
+            return p.ps_i64 ? static_cast<const int64_t*>(p.pslots)[at]
+                            : static_cast<int64_t>(static_cast<const int32_t*>(p.pslots)[at]);
+        }
+        return p.tables[static_cast<int64_t>(b.r) * p.t_s0 + (pow2 ? pos >> bshift : pos / B)];   // the page
+    };
+    const int64_t s0 = (g ? p.v_s0 : p.k_s0) * static_cast<int64_t>(sizeof(T));
+    const int64_t s1 = (g ? p.v_s1 : p.k_s1) * static_cast<int64_t>(sizeof(T));
+    const uint64_t head0 = reinterpret_cast<uint64_t>(g ? p.v : p.k) +
+                           static_cast<uint64_t>(kvh * (g ? p.v_s2 : p.k_s2) * static_cast<int64_t>(sizeof(T)));
+    // The tile's K and V row addresses into the wave's LDS list; returns the tile's present keys,
+    // one bit each.
+    auto resolve = [&](int t0, int64_t s, int buf) __attribute__((always_inline)) -> uint32_t {
+        const int pos = t0 + c;
+        int64_t blk = 0, off = 0;
+        bool ok = false;
+        if (pos < b.seq) {
+            if (pos < P && !p.pslots) {
+                blk = s;
+                off = pow2 ? pos & (B - 1) : pos % B;
+                ok = s >= 0 && s < p.num_blocks;
+            } else {
+                ok = s >= 0 && s < pool_slots;
+                if (static_cast<uint64_t>(s) < (1ull << 32)) {
+                    blk = static_cast<uint32_t>(s) / static_cast<uint32_t>(B);
+                } else {
+                    blk = ok ? s / B : 0;
+                }
+                off = s - blk * B;
+            }
+            if (!ok && g == 0) set_status(p.status, TV_STATUS_BAD_PAGE);
+        }
+        // A missing key reads the pool's first row: its score is hidden, and the loads need no
+        // conditions.
+        uint64_t at = head0;
+        if (ok) at += static_cast<uint64_t>(blk * s0 + off * s1);
+        rows_lds[wave][buf][g][c] = at;
+        return static_cast<uint32_t>(__ballot(ok));
+    };
+
+    // K operand registers of one slab: 16 bytes per step (f32: dims 8j + 4g, 16-bit: 16j + 8g).
+    u32x4 kr[KV4];
+    auto k_load = [&](int buf, int slab) __attribute__((always_inline)) {
+        const uint64_t at = rows_lds[wave][buf][0][c];
+        const T* k = reinterpret_cast<const T*>(at) + (KSTEP / 2) * g;
+#pragma unroll
+        for (int j = 0; j < KV4; ++j) {
+            const int d = SLAB * slab + KSTEP * j;
+            if (EXACT ? d < DIM : d < D) {
+                if (EXACT || p.vec) {
+                    kr[j] = *reinterpret_cast<const u32x4*>(k + d);
+                } else {
+                    T e[16 / sizeof(T)];
+                    const int dl = d + (KSTEP / 2) * opaque(g);
+                    const T* row = reinterpret_cast<const T*>(at);
+#pragma unroll
+                    for (int i = 0; i < static_cast<int>(16 / sizeof(T)); ++i) {
+                        e[i] = dl + i < D ? row[(dl + i) * p.k_s3] : static_cast<T>(0.f);
+                    }
+                    kr[j] = __builtin_bit_cast(u32x4, e);
+                }
+            }
+        }
+    };
+    // V operand registers of one slab: for S^T register r the two dims 64j + 2c, + 1 of its key
+    // (past D: the last ones again, for output dims that are not stored).
+    typedef typename std::conditional<F32, u32x2, uint32_t>::type VPair;
+    VPair vr[16][SB];
+    auto v_load = [&](int buf, int slab) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const T* v = reinterpret_cast<const T*>(rows_lds[wave][buf][1][8 * (r >> 2) + 4 * g + (r & 3)]);
+#pragma unroll
+            for (int j = 0; j < SB; ++j) {
+                const int d0 = SLAB * slab + 64 * j;
+                if (EXACT ? d0 < DIM : d0 < D) {
+                    if (EXACT || p.vec) {
+                        vr[r][j] = *reinterpret_cast<const VPair*>(v + (EXACT && d0 + 64 <= DIM ? d0 + 2 * c
+                                                                                                : min(d0 + 2 * c, D - 2)));
+                    } else {
+                        const int d = d0 + 2 * opaque(c);
+                        T e[2];
+                        e[0] = v[min(d, D - 1) * p.v_s3];
+                        e[1] = v[min(d + 1, D - 1) * p.v_s3];
+                        vr[r][j] = __builtin_bit_cast(VPair, e);
+                    }
+                }
+            }
+        }
+    };
+
+    f32x16 acc[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) acc[i] = f32x16{};
+    float m = -INFINITY, l = 0.f;
+
+    // V values that are not finite would reach rows the product multiplies by zero (keys hidden
+    // from a row) or, split into three terms, turn an infinity into a NaN: such keys leave the
+    // operand and are added one at a time, to the rows that give them weight.
+    auto finite_v = [&](const f32x16& pr, int buf, int slab) __attribute__((always_inline)) {
+        // Magnitude bits of a pair: two words (f32) or two halves of one.
+        typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+        typedef typename std::conditional<F32, uint32_t, u16x2>::type Mag;
+        constexpr uint32_t kInf = F32 ? 0x7f800000u : (std::is_same<T, __bf16>::value ? 0x7f80u : 0x7c00u);
+        auto magnitude = [&](int r, int j) __attribute__((always_inline)) -> Mag {
+            if constexpr (F32) return max(vr[r][j][0] & 0x7fffffffu, vr[r][j][1] & 0x7fffffffu);
+            else return __builtin_bit_cast(u16x2, vr[r][j] & 0x7fff7fffu);
+        };
+        auto over = [&](Mag x) __attribute__((always_inline)) -> bool {
+            if constexpr (F32) return x >= kInf;
+            else return x[0] >= kInf || x[1] >= kInf;
+        };
+        Mag top = magnitude(0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+#pragma unroll
+            for (int j = 0; j < SB; ++j) {
+                if (EXACT ? SLAB * slab + 64 * j < DIM : SLAB * slab + 64 * j < D) {
+                    top = __builtin_elementwise_max(top, magnitude(r, j));
+                }
+            }
+        }
+        if (!__any(over(top))) return;
+        uint32_t bad = 0;   // the tile's keys with such a value
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            bool here = false;
+#pragma unroll
+            for (int j = 0; j < SB; ++j) here |= SLAB * slab + 64 * j < D && over(magnitude(r, j));
+            const uint64_t both = __ballot(here);
+            const int key = 8 * (r >> 2) + (r & 3);
+            if (both & 0xffffffffull) bad |= 1u << key;
+            if (both >> 32) bad |= 1u << (key + 4);
+            if (g ? (both >> 32) != 0 : (both & 0xffffffffull) != 0) {
+#pragma unroll
+                for (int j = 0; j < SB; ++j) vr[r][j] = VPair{};
+            }
+        }
+        for (; bad; bad &= bad - 1) {
+            const int key = __builtin_ctz(bad), reg = 4 * (key >> 3) + (key & 3), half = (key >> 2) & 1;
+            float w = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) w = r == reg ? pr[r] : w;
+            w = __shfl(w, c + 32 * half);
+            const T* v = reinterpret_cast<const T*>(rows_lds[wave][buf][1][key]);
+            const int d0 = opaque(8 * g);
+#pragma unroll
+            for (int n = 0; n < SLAB / 32; ++n) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int d = d0 + SLAB * slab + 64 * (n >> 1) + 16 * (r >> 2) + 2 * (r & 3) + (n & 1);
+                    const float x = to_float(v[min(d, D - 1) * p.v_s3]);
+                    acc[SLAB / 32 * slab + n][r] += w != 0.f ? w * x : 0.f;
+                }
+            }
+        }
+    };
+
+    // Software pipeline of a wave: while tile i is computed, its V loads, the K loads of its next
+    // tile and the slot lookup of the one after are in flight.
+    const int first = tbeg + wave;
+    // A pool without pages has no row to read: the rows come out empty.
+    const bool empty = p.num_blocks < 1;
+    if (empty && tid == 0) set_status(p.status, TV_STATUS_BAD_PAGE);
+    const int count = first < tend && !empty ? (tend - first + kWaves - 1) / kWaves : 0;
+    int64_t next_slot = count > 0 ? slot_load(kTile * first) : -1;
+    // Q block into LDS (zeros past the block's rows and past D): eight threads a row.
+    {
+        const int rr = tid >> 3, part = tid & 7;
+        constexpr int PER = 16 / sizeof(T), LOADS = (DP + 8 * PER - 1) / (8 * PER);
+        const bool here = rr < b.rows;
+        const int node = (b.row0 + rr) / G, head = kvh * G + (b.row0 + rr) - node * G;
+        const T* q = static_cast<const T*>(p.q) +
+                     (here ? (b.tree0 + node) * p.q_s0 + static_cast<int64_t>(head) * p.q_s1 : 0);
+        u32x4 x[LOADS];
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int d = PER * (8 * i + part);
+            x[i] = u32x4{0u, 0u, 0u, 0u};
+            if (p.q_vec) {
+                if (here && d < D) x[i] = *reinterpret_cast<const u32x4*>(q + d);
+            } else {
+                T e[PER];
+#pragma unroll
+                for (int n = 0; n < PER; ++n) e[n] = here && d + n < D ? q[d + n] : static_cast<T>(0.f);
+                x[i] = __builtin_bit_cast(u32x4, e);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int d = PER * (8 * i + part);
+            if (d < DP) *reinterpret_cast<u32x4*>(smem + rr * QPITCH + d * static_cast<int>(sizeof(T)) / 4) = x[i];
+        }
+    }
+    // The metadata must place a request's rows consecutively.
+    bool row_ok = in_block;
+    if (row_request != b.r || row_local != local) {
+        set_status(p.status, TV_STATUS_BAD_REQUEST);
+        row_ok = false;
+    }
+    const int my_end = row_ok ? P + local + 1 : 0;         // this row's visible range
+    const float* bias_row = p.bias + (row_ok ? bias_base + static_cast<int64_t>(local) * b.nodes : 0);
+    uint32_t valid = 0;
+    if (count > 0) {
+        valid = resolve(kTile * first, next_slot, 0);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wave's own list
+        k_load(0, 0);
+        if (count > 1) next_slot = slot_load(kTile * (first + kWaves));
+    }
+    __syncthreads();   // Q staged
+    for (int i = 0; i < count; ++i) {
+        const int t0 = kTile * (first + kWaves * i), buf = i & 1;
+        const uint32_t here = valid;
+        v_load(buf, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        // Scores.
+        f32x16 s = f32x16{};
+#pragma unroll
+        for (int slab = 0; slab < SLABS; ++slab) {
+            if (slab > 0) k_load(buf, slab);
+#pragma unroll
+            for (int j = 0; j < KV4; ++j) {
+                if (EXACT ? SLAB * slab + KSTEP * j < DIM : SLAB * slab + KSTEP * j < D) {
+                    const u32x4 qw = *reinterpret_cast<const u32x4*>(
+                        smem + c * QPITCH + (F32 ? SLAB * slab + 8 * j + 4 * g : (SLAB * slab + 16 * j + 8 * g) / 2));
+                    if constexpr (F32) {
+                        const f32x4 a = __builtin_bit_cast(f32x4, kr[j]), q4 = __builtin_bit_cast(f32x4, qw);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], q4[e], s, 0, 0, 0);
+                    } else {
+                        typedef typename Op<T>::vec V8;
+                        s = Op<T>::mfma(__builtin_bit_cast(V8, kr[j]), __builtin_bit_cast(V8, qw), s);
+                    }
+                }
+            }
+        }
+        if (i + 1 < count) {
+            valid = resolve(t0 + kTile * kWaves, next_slot, buf ^ 1);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            k_load(buf ^ 1, 0);
+            if (i + 2 < count) next_slot = slot_load(t0 + 2 * kTile * kWaves);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // Softmax of the 16 keys this lane holds (key 8 * (r / 4) + 4 * g + r % 4).
+        const bool masked = here != ~0u || t0 + kTile > P;
+        const float mul = masked ? 1.f : cs;   // masked tiles hold finished scores, the others K.Q
+        float mx = -INFINITY;
+        if (masked) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = 8 * (r >> 2) + 4 * g + (r & 3), pos = t0 + key;
+                bool visible = pos < my_end && ((here >> key) & 1u);
+                float x = s[r] * cs;
+                if (visible && pos >= P) {
+                    const float bias = bias_row[pos - P];
+                    visible = bias != -INFINITY;
+                    x = fmaf(bias, kLog2eF, x);
+                }
+                s[r] = visible ? x : -INFINITY;
+                mx = fmaxf(mx, s[r]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r] * cs);
+        }
+        if (__any(mx > m + kRaiseMargin)) {   // rare after the first tile
+            // Both halves of a row decide on the whole row; rows that do not ask keep their maximum.
+            const float row_max = fmaxf(mx, __shfl_xor(mx, 32));
+            if (row_max > m + kRaiseMargin) {
+                const float alpha = __builtin_amdgcn_exp2f(m - row_max);   // 0 while m is -inf
+                l *= alpha;
+#pragma unroll
+                for (int n = 0; n < NB; ++n) acc[n] *= alpha;
+                m = row_max;
+            }
+        }
+        const float ref = m == -INFINITY ? 0.f : Op<T>::kShift - m;   // a score of -inf gives 0, whatever m
+        float l0 = 0.f, l1 = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float pr = __builtin_amdgcn_exp2f(fmaf(s[r], mul, ref));
+            s[r] = pr;
+            if (r & 1) l1 += pr; else l0 += pr;
+        }
+        l += l0 + l1;
+        // P.V.
+#pragma unroll
+        for (int slab = 0; slab < SLABS; ++slab) {
+            if (!EXACT && SLAB * slab >= D) continue;
+            if (slab > 0) v_load(buf, slab);
+            // f32: a key that no row of a tile is denied needs no care, its infinities and NaNs enter
+            // as they would one key at a time.
+            if (!F32 || masked) finite_v(s, buf, slab);
+#pragma unroll
+            for (int j = 0; j < SB; ++j) {
+                if (EXACT ? SLAB * slab + 64 * j < DIM : SLAB * slab + 64 * j < D) {
+                    f32x16& even = acc[SLAB / 32 * slab + 2 * j];
+                    f32x16& odd = acc[SLAB / 32 * slab + 2 * j + 1];
+                    if constexpr (F32) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const f32x2 a = __builtin_bit_cast(f32x2, vr[r][j]);
+                            even = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], s[r], even, 0, 0, 0);
+                            odd = __builtin_amdgcn_mfma_f32_32x32x2f32(a[1], s[r], odd, 0, 0, 0);
+                        }
+                    } else {
+                        typedef typename Op<T>::vec V8;
+#pragma unroll
+                        for (int kk = 0; kk < 2; ++kk) {
+                            V8 hi, mid, lo;
+                            uint32_t we[4], wo[4];
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) {
+                                const float pr = s[8 * kk + e];
+                                hi[e] = static_cast<T>(pr);
+                                const float r1 = pr - static_cast<float>(hi[e]);
+                                mid[e] = static_cast<T>(r1);
+                                lo[e] = static_cast<T>(r1 - static_cast<float>(mid[e]));
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const uint32_t x = vr[8 * kk + 2 * e][j], y = vr[8 * kk + 2 * e + 1][j];
+                                we[e] = __builtin_amdgcn_perm(y, x, 0x05040100u);   // low halves of x, y
+                                wo[e] = __builtin_amdgcn_perm(y, x, 0x07060302u);   // high halves
+                            }
+                            const V8 ae = __builtin_bit_cast(V8, we), ao = __builtin_bit_cast(V8, wo);
+                            even = Op<T>::mfma(ae, lo, even);
+                            odd = Op<T>::mfma(ao, lo, odd);
+                            even = Op<T>::mfma(ae, mid, even);
+                            odd = Op<T>::mfma(ao, mid, odd);
+                            even = Op<T>::mfma(ae, hi, even);
+                            odd = Op<T>::mfma(ao, hi, odd);
+                        }
+                    }
+                }
+            }
+        }
+    }
+
+    // Merge of the four waves' softmaxes: the row's maximum and sum, then the O rows in LDS.
+    l += __shfl_xor(l, 32);
+    if (g == 0) ml_lds[wave][c] = make_float2(m, l);
+    __syncthreads();   // every wave is past its Q reads
+    float row_m = ml_lds[0][c].x;
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) row_m = fmaxf(row_m, ml_lds[w][c].x);
+    const float scale_w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - row_m);
+    float* o_lds = reinterpret_cast<float*>(smem);
+    // acc block 2j + i, register r of half g: dim 64j + 2 * (8 * (r / 4) + 4 * g + r % 4) + i.
+    auto o_at = [&](int buf, int j, int r) __attribute__((always_inline)) -> f32x2* {
+        return reinterpret_cast<f32x2*>(o_lds + buf * O_WORDS + c * OPITCH + 64 * j +
+                                        2 * (8 * (r >> 2) + 4 * g + (r & 3)));
+    };
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[n] *= scale_w;
+    auto put = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NB / 2; ++j) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) *o_at(buf, j, r) = f32x2{acc[2 * j][r], acc[2 * j + 1][r]};
+        }
+    };
+    auto take = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NB / 2; ++j) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const f32x2 x = *o_at(buf, j, r);
+                acc[2 * j][r] += x[0];
+                acc[2 * j + 1][r] += x[1];
+            }
+        }
+    };
+    if (wave >= 2) put(wave - 2);
+    __syncthreads();
+    if (wave < 2) take(wave);
+    if (wave == 1) put(1);   // its own buffer: only wave 1 read it
+    __syncthreads();
+    if (wave == 0) {
+        take(1);
+        put(0);
+    }
+    __syncthreads();
+    const bool split = b.tiles > b.chunk;   // this block has further chunks
+    const int64_t part = ((b.number * p.kv_heads + kvh) * p.splits + b.part) * kBlockRows;
+    if (split && tid < kBlockRows) {
+        float sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const float2 x = ml_lds[w][tid];
+            sum += x.x == -INFINITY ? 0.f : x.y * __builtin_amdgcn_exp2f(x.x - row_m);
+        }
+        p.ws_ml[part + tid] = make_float2(row_m, sum);   // tid < 32: lane tid holds row tid's maximum
+    }
+    for (int rr = tid / kWave; rr < b.rows; rr += kWaves) {
+        float inv = 0.f;
+        int64_t base = 0;
+        if (!split) {
+            float top = ml_lds[0][rr].x, sum = 0.f;
+#pragma unroll
+            for (int w = 1; w < kWaves; ++w) top = fmaxf(top, ml_lds[w][rr].x);
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                const float2 x = ml_lds[w][rr];
+                sum += x.x == -INFINITY ? 0.f : x.y * __builtin_amdgcn_exp2f(x.x - top);
+            }
+            inv = 1.f / sum;
+            const int node = (b.row0 + rr) / G, head = kvh * G + (b.row0 + rr) % G;
+            const int64_t at = b.tree0 + node;
+            if (p.q2r[at] != b.r || p.local[at] != node) continue;   // reported above
+            base = at * p.o_s0 + static_cast<int64_t>(head) * p.o_s1;
+        }
+        for (int d = lane; d < D; d += kWave) {
+            const float x = o_lds[rr * OPITCH + d];
+            if (split) {
+                p.ws_o[(part + rr) * D + d] = x;
+            } else {
+                store_value(p, base + d, x * inv);
+            }
+        }
+    }
+}
+
+template <typename T, int DIM, bool EXACT>
+__global__ void __launch_bounds__(kThreadsFp32, DIM <= 128 ? 2 : 1)
+tree_attention_fp32_kernel(const Fp32Params p) {
+    // Index -> (block, chunk) and KV head, head fastest: with 8 KV heads the blocks and chunks of one
+    // head share an XCD (workgroup i runs on XCD i % 8), and so its K/V in that L2.
+    RowBlock b;
+    if (p.splits == 1) {
+        const int64_t unit = p.unit0 + blockIdx.x;
+        const int64_t number = unit / p.kv_heads;
+        const int r = __builtin_amdgcn_readfirstlane(request_of_group(p.cu, p.groups, p.num_requests, number));
+        const int index = __builtin_amdgcn_readfirstlane(static_cast<int>(number - group_start(p.cu, p.groups, r)));
+        if (block_of_request(p, r, index, p.cu[r], p.cnt[r], p.plen[r], b, true)) {
+            attend_block<T, DIM, EXACT>(p, b, static_cast<int>(unit - number * p.kv_heads));
+        }
+        return;
+    }
+    const Cut cut = plan_cut(p);
+    for (int i = blockIdx.x;; i += gridDim.x) {
+        const int u = i / p.kv_heads;
+        bool live;
+        if (!cut_block(p, cut, u, b, live)) return;
+        if (live) {
+            attend_block<T, DIM, EXACT>(p, b, i - u * p.kv_heads);
+            __syncthreads();   // the next block reuses the LDS
+        }
+    }
+}
+
+// Combines the chunks of the row blocks that were cut: one wave per score row, its partial
+// rows read coalesced and all in flight together.
+__global__ void __launch_bounds__(kThreadsFp32)
+merge_fp32_kernel(const Fp32Params p) {
+    const Cut cut = plan_cut(p);
+    const int number = blockIdx.x / p.kv_heads, kvh = blockIdx.x % p.kv_heads;
+    const int lane = threadIdx.x & (kWave - 1);
+    // The request whose numbers hold this one: the last that starts at or before it.
+    const bool before = lane < p.num_requests &&
+                        static_cast<int64_t>(cut.cu) * p.groups / kBlockRows + lane <= number;
+    const int r = 63 - __builtin_clzll(__ballot(before) | 1ull);
+    const int cu = __builtin_amdgcn_readlane(cut.cu, r), tiles = __builtin_amdgcn_readlane(cut.tiles, r);
+    RowBlock b;
+    if (!block_of_request(p, r, number - static_cast<int>(static_cast<int64_t>(cu) * p.groups / kBlockRows + r), cu,
+                          __builtin_amdgcn_readlane(cut.nodes, r), __builtin_amdgcn_readlane(cut.prefix, r), b, false) ||
+        tiles == 0) {
+        return;
+    }
+    const int chunk = chunk_tiles(tiles, chunks_of(tiles, cut.target));
+    if (b.tiles <= chunk) return;   // one chunk: the attention kernel wrote the rows
+    const int parts = (b.tiles + chunk - 1) / chunk;
+    const int64_t first = (b.number * p.kv_heads + kvh) * p.splits * kBlockRows;
+    const int rr = blockIdx.y * kWaves + threadIdx.x / kWave;
+    if (rr >= b.rows) return;
+    const int node = (b.row0 + rr) / p.groups, head = kvh * p.groups + (b.row0 + rr) % p.groups;
+    const int64_t at = b.tree0 + node;
+    if (p.q2r[at] != r || p.local[at] != node) return;
+    // Lane s holds partial s's maximum and sum.
+    const float2 ml = lane < parts ? p.ws_ml[first + lane * kBlockRows + rr] : make_float2(-INFINITY, 0.f);
+    float top = ml.x;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+    const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - top);
+    float sum = ml.y * w;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    const float inv = 1.f / sum;
+    const int64_t base = at * p.o_s0 + static_cast<int64_t>(head) * p.o_s1;
+    for (int d0 = 0; d0 < p.head_dim; d0 += kWave) {   // every lane takes part in the exchange
+        const int d = d0 + lane, dl = min(d, p.head_dim - 1);
+        float o = 0.f;
+#pragma unroll
+        for (int s0 = 0; s0 < kMaxSplits; s0 += 8) {
+            float x[8];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                x[s] = s0 + s < parts ? p.ws_o[(first + (s0 + s) * kBlockRows + rr) * p.head_dim + dl] : 0.f;
+            }
+#pragma unroll
+            for (int s = 0; s < 8; ++s) o = fmaf(x[s], __shfl(w, s0 + s), o);   // w is 0 past the parts
+        }
+        if (d < p.head_dim) store_value(p, base + d, o * inv);
+    }
+}
+
+// Row-block numbers of a launch (group_start) and the chunks its blocks may be cut into, from
+// the launch's shapes alone: a batch of kCutRows row blocks or more is not cut.
+int64_t row_groups(int64_t total_queries, int64_t num_requests, int64_t groups) {
+    return total_queries * groups / kBlockRows + num_requests + 1;
+}
+int split_count(int64_t total_queries, int64_t num_requests, int64_t groups, int64_t kv_heads) {
+    const int64_t units = row_groups(total_queries, num_requests, groups) * kv_heads;
+    if (num_requests > kCutRequests) return 1;
+    return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, kCutRows / units)));
+}
+int64_t partial_bytes(int64_t units, int splits, int32_t head_dim) {
+    return units * splits * kBlockRows * (static_cast<int64_t>(head_dim) * 4 + static_cast<int64_t>(sizeof(float2)));
+}
+
+// Rows the vector loads take: unit element stride, 16-byte aligned rows, and a head size
+// that divides into steps of two 16-byte pieces (one per lane half).
+bool vector_rows(const void* base, const int64_t* stride, int64_t elem, int32_t head_dim) {
+    const int64_t per = 16 / elem;
+    return stride[3] == 1 && head_dim % (2 * per) == 0 && aligned(base, 16) && stride[0] % per == 0 &&
+           stride[1] % per == 0 && stride[2] % per == 0;
+}
+
+template <typename T, int DIM, bool EXACT>
+void launch_for_dims(const Fp32Params& p, const dim3& grid, hipStream_t s) {
+    hipLaunchKernelGGL((tree_attention_fp32_kernel<T, DIM, EXACT>), grid, dim3(kThreadsFp32), 0, s, p);
+}
+
+// The head sizes models use are compiled in; the others share an instance per power of two.
+template <typename T>
+void launch_for_type(const Fp32Params& p, uint32_t units, hipStream_t s) {
+    // Cut: the blocks' first chunks and the chip's slots; workgroups loop where that is too few.
+    const dim3 grid(p.splits == 1 ? units : units + p.slots);
+    const int d = p.head_dim;
+    if (p.vec && d == 64) {
+        launch_for_dims<T, 64, true>(p, grid, s);
+    } else if (p.vec && d == 80) {
+        launch_for_dims<T, 80, true>(p, grid, s);
+    } else if (p.vec && d == 96) {
+        launch_for_dims<T, 96, true>(p, grid, s);
+    } else if (p.vec && d == 112) {
+        launch_for_dims<T, 112, true>(p, grid, s);
+    } else if (p.vec && d == 128) {
+        launch_for_dims<T, 128, true>(p, grid, s);
+    } else if (p.vec && d == 192) {
+        launch_for_dims<T, 192, true>(p, grid, s);
+    } else if (p.vec && d == 256) {
+        launch_for_dims<T, 256, true>(p, grid, s);
+    } else if (d <= 64) {
+        launch_for_dims<T, 64, false>(p, grid, s);
+    } else if (d <= 128) {
+        launch_for_dims<T, 128, false>(p, grid, s);
+    } else if (d <= 256) {
+        launch_for_dims<T, 256, false>(p, grid, s);
     } else {
-        launch_for_dims<T, 8>(p, grid, s);
+        launch_for_dims<T, 512, false>(p, grid, s);
+    }
+    if (p.splits > 1) {
+        hipLaunchKernelGGL(merge_fp32_kernel, dim3(units, kBlockRows / kWaves), dim3(kThreadsFp32), 0, s,
+                           p);
     }
 }
 
@@ -406,7 +952,22 @@ using namespace tv;
 
 extern "C" int64_t tv_sizeof_tree_attention_fp32_args(void) { return sizeof(tv_tree_attention_fp32_args); }
 
+extern "C" int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries, int32_t num_requests,
+                                                          int32_t num_q_heads, int32_t num_kv_heads,
+                                                          int32_t head_dim) {
+    if (total_queries < 1 || num_requests < 1 || num_kv_heads < 1 || num_q_heads < num_kv_heads || head_dim < 1) return 0;
+    const int64_t groups = num_q_heads / num_kv_heads;
+    const int splits = split_count(total_queries, num_requests, groups, num_kv_heads);
+    if (splits == 1) return 0;
+    return partial_bytes(row_groups(total_queries, num_requests, groups) * num_kv_heads, splits, head_dim);
+}
+
 extern "C" int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* a, void* stream) {
+    return tv_tree_attention_fp32_split(a, nullptr, 0, stream);
+}
+
+extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a, void* workspace,
+                                            int64_t workspace_bytes, void* stream) {
     clear_error();
     if (!a) return fail(TV_ERR_INVALID, "tree_attention_fp32: null args");
     if (a->num_requests < 1 || a->total_queries < 0) return fail(TV_ERR_INVALID, "tree_attention_fp32: invalid counts");
@@ -415,6 +976,8 @@ extern "C" int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* a, void
                     a->num_kv_heads);
     }
     if (a->num_kv_heads > 65535) return fail(TV_ERR_UNSUPPORTED, "tree_attention_fp32: more than 65535 KV heads");
+    const int64_t units = row_groups(a->total_queries, a->num_requests, a->num_q_heads / a->num_kv_heads) *
+                          a->num_kv_heads;
     if (a->head_dim < 1 || a->head_dim > 512) {
         return fail(TV_ERR_UNSUPPORTED, "tree_attention_fp32: head_dim %d (implemented: 1..512)", a->head_dim);
     }
@@ -471,15 +1034,45 @@ extern "C" int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* a, void
     p.groups = a->num_q_heads / a->num_kv_heads;
     p.head_dim = a->head_dim;
     p.block_size = a->block_size;
-    p.scale = a->scale;
+    p.scale = a->scale * kLog2eF;
     p.status = a->status;
+    p.kv_heads = a->num_kv_heads;
+    p.splits = 1;
+    p.ws_o = nullptr;
+    p.ws_ml = nullptr;
+    if (workspace) {
+        const int splits = split_count(a->total_queries, a->num_requests, p.groups, a->num_kv_heads);
+        if (splits > 1) {
+            if (!aligned(workspace, 16)) return fail(TV_ERR_INVALID, "tree_attention_fp32: unaligned workspace");
+            if (workspace_bytes < partial_bytes(units, splits, a->head_dim)) {
+                return fail(TV_ERR_CAPACITY, "tree_attention_fp32: workspace of %lld bytes, %lld needed",
+                            (long long)workspace_bytes, (long long)partial_bytes(units, splits, a->head_dim));
+            }
+            p.splits = splits;
+            p.slots = a->head_dim <= 128 ? 2 * kCus : kCus;   // the kernel's launch bounds
+            p.min_chunk = a->in_dtype == TV_F32 ? kMinChunk32 : kMinChunk16;
+            // (maximum, sum) pairs first: 8-byte aligned whatever the head size.
+            p.ws_ml = static_cast<float2*>(workspace);
+            p.ws_o = reinterpret_cast<float*>(p.ws_ml + units * splits * kBlockRows);
+        }
+    }
     hipStream_t s = as_stream(stream);
-    if (a->in_dtype == TV_F32) {
-        launch_for_type<float>(p, a->num_kv_heads, s);
-    } else if (a->in_dtype == TV_BF16) {
-        launch_for_type<__bf16>(p, a->num_kv_heads, s);
-    } else {
-        launch_for_type<_Float16>(p, a->num_kv_heads, s);
+    const int64_t elem = a->in_dtype == TV_F32 ? 4 : 2;
+    p.vec = vector_rows(a->k_pool, a->k_stride, elem, a->head_dim) &&
+            vector_rows(a->v_pool, a->v_stride, elem, a->head_dim);
+    const int64_t per = 16 / elem;
+    p.q_vec = aligned(a->q, 16) && a->q_stride_row % per == 0 && a->q_stride_head % per == 0 && a->head_dim % per == 0;
+    // A grid holds 2^32 threads: a huge batch takes several launches.
+    constexpr int64_t kLaunchUnits = int64_t{1} << 23;
+    for (p.unit0 = 0; p.unit0 < units; p.unit0 += kLaunchUnits) {
+        const uint32_t count = static_cast<uint32_t>(std::min(kLaunchUnits, units - p.unit0));
+        if (a->in_dtype == TV_F32) {
+            launch_for_type<float>(p, count, s);
+        } else if (a->in_dtype == TV_BF16) {
+            launch_for_type<__bf16>(p, count, s);
+        } else {
+            launch_for_type<_Float16>(p, count, s);
+        }
     }
     return check_launch("tree_attention_fp32");
 }

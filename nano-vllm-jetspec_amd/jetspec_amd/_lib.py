@@ -61,6 +61,8 @@ EXPORTED_SYMBOLS = (
     "tv_tree_attention_workspace_bytes",
     "tv_tree_attention_fp32",
     "tv_sizeof_tree_attention_fp32_args",
+    "tv_tree_attention_fp32_split",
+    "tv_tree_attention_fp32_workspace_bytes",
 )
 
 
@@ -226,6 +228,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tv_tree_attention_workspace_bytes.argtypes = [c_int32, c_int32]
     lib.tv_tree_attention_fp32.restype = c_int32
     lib.tv_tree_attention_fp32.argtypes = [POINTER(TreeAttentionFp32Args), c_void_p]
+    lib.tv_tree_attention_fp32_split.restype = c_int32
+    lib.tv_tree_attention_fp32_split.argtypes = [POINTER(TreeAttentionFp32Args), c_void_p, c_int64, c_void_p]
+    lib.tv_tree_attention_fp32_workspace_bytes.restype = c_int64
+    lib.tv_tree_attention_fp32_workspace_bytes.argtypes = [c_int32] * 5
     lib.tv_sizeof_tree_attention_fp32_args.restype = c_int64
     lib.tv_sizeof_tree_attention_fp32_args.argtypes = []
     lib.tv_sizeof_rope_scatter_args.restype = c_int64

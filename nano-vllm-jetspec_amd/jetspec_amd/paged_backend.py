@@ -171,6 +171,18 @@ def _fp32_template(metadata, k_pool, v_pool, queries_per_kv: int, device):
     return a
 
 
+def _enqueue_fp32(a, device, stream: int, what: str) -> None:
+    """Launch a complete FP32-kernel block.  A batch of few score rows cuts its keys over several
+    workgroups through a workspace that lives for this call only, as any temporary of the
+    stream (or of the graph being captured): no two launches share one."""
+    lib = _lib.library()
+    size = int(lib.tv_tree_attention_fp32_workspace_bytes(a.total_queries, a.num_requests, a.num_q_heads,
+                                                          a.num_kv_heads, a.head_dim))
+    workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
+    _lib.check(lib.tv_tree_attention_fp32_split(ctypes.byref(a), workspace.data_ptr() if size else None, size, stream),
+               what)
+
+
 def _launch_fp32(a, q, out, scale, stream: int) -> torch.Tensor:
     """Complete a copy of an FP32-kernel argument block with Q, O and scale, and launch."""
     a = _lib.TreeAttentionFp32Args.from_buffer_copy(a)
@@ -182,7 +194,7 @@ def _launch_fp32(a, q, out, scale, stream: int) -> torch.Tensor:
     a.out_stride_row, a.out_stride_head = out.stride(0), out.stride(1)
     a.out_dtype = _device.dtype_code(out.dtype)
     a.scale = float(scale)
-    _lib.check(_lib.library().tv_tree_attention_fp32(ctypes.byref(a), stream), "tree_attention_fp32")
+    _enqueue_fp32(a, q.device, stream, "tree_attention_fp32")
     return out
 
 
@@ -570,8 +582,7 @@ def _legacy_fp32(q, k_pool, v_pool, req, scale, block_size: int, out, device) ->
     a.block_size = block_size
     a.scale = float(scale)
     a.status = _device.status_word(device).data_ptr()
-    _lib.check(_lib.library().tv_tree_attention_fp32(ctypes.byref(a), _device.stream_handle(device)),
-               "tree_attention_fp32 (slot addressed)")
+    _enqueue_fp32(a, device, _device.stream_handle(device), "tree_attention_fp32 (slot addressed)")
 
 
 def _legacy_mfma(q, k_pool, v_pool, req, scale, num_queries_per_kv: int, block_size: int, out, device) -> None:
