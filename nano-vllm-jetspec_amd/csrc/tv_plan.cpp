@@ -9,11 +9,9 @@
 // so a KV tile staged in LDS is reused by every (node, query head) row of its group.
 // Long prefixes are cut into chunks (split-K) only as far as needed to give every
 // compute unit work; items are ordered longest first so the hardware dispatcher's
-// greedy assignment balances ragged contexts (an LPT schedule).  When that chunking
-// leaves a few rounds of items with the last round part-empty (more items than compute
-// units, at most kFillRounds rounds), the chunk target is lowered to the smallest
-// value whose item count still fits the same number of full rounds, so the rounds
-// fill with smaller, more even chunks.
+// greedy assignment balances ragged contexts (an LPT schedule).  Up to kFillRounds
+// rounds of items, the chunk target is the smallest whose items fit a chosen number of
+// whole rounds (see kRoundCost), so no round is part-empty.
 #include <stdint.h>
 
 #include <algorithm>
@@ -32,7 +30,35 @@ constexpr int kMaxChunkPages = 512; // page numbers a workgroup caches in LDS
 constexpr int kMaxSlotChunk = 2048; // prefix slots a workgroup caches in LDS (slot addressing)
 constexpr int kMaxTreeNodes = 2048; // tree slots a workgroup caches in LDS (page-table prefixes)
 constexpr int kMaxTreeNodesSlots = 1024;   // ... beside a slot-addressed prefix chunk
-constexpr int64_t kFillRounds = 4;  // item rounds the chunk target is refitted for
+constexpr int64_t kFillRounds = 4;  // item rounds the chunk target is chosen for
+
+// Choice of the chunk target, in cost units (about 142 a microsecond).  A batch that fits one
+// round gets as many items as balance its streaming against its partial results: n items of
+// an even share stream total / n, and each writes and the merge reads 133 KB, about
+// kPartialCost, so n = sqrt(total / kPartialCost), at most one per compute unit.  A batch that
+// does not fit one round when every item has the even share of a compute unit takes the number
+// of whole rounds whose estimated span is the smallest: a round costs its longest item and
+// kRoundCost (the item's lookups, first loads and stores, 8 us), a slot kSlotCost (what of its
+// merge the launch does not hide).  8 requests of 1354-4060 keys and 18-54 nodes, 8 KV heads:
+// 496 items in two rounds 64.5 us, 244 in one 49.1; a one-head shard of 32 requests of
+// 1.1k-8.1k keys: 499 items 75.8 us, 227 items 53.9; 8 requests of 545-1603 keys and 32 nodes:
+// 236 items 29.9 us, 160 items 27.9.
+constexpr int64_t kPartialCost = 8;
+constexpr int64_t kRoundCost = 1000;
+constexpr int64_t kSlotCost = 2;
+constexpr int64_t kTauStep = 128;   // 32 keys of a one-head item
+
+int64_t one_round_items(int64_t total_cost, int64_t units, int64_t compute_units) {
+    const int64_t x = total_cost / kPartialCost;
+    int64_t n = compute_units;
+    if (x < compute_units * compute_units) {
+        n = 0;
+        for (int64_t bit = int64_t{1} << 20; bit > 0; bit >>= 1) {   // integer square root
+            if ((n + bit) * (n + bit) <= x) n += bit;
+        }
+    }
+    return std::min(compute_units, std::max(n, units));
+}
 
 struct Item {
     int32_t r, h0, n0, kbeg, kend, flags, slot, hpw;
@@ -178,7 +204,7 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
         return fail(TV_ERR_INVALID, "plan: chunk_keys %d must be a non-negative multiple of 32", chunk_keys);
     }
     int32_t max_nodes = 1;
-    int64_t total_cost = 0;
+    int64_t total_cost = 0, units = 0;
     for (int32_t r = 0; r < num_requests; ++r) {
         const int32_t p = prefix_lens_host[r], t = node_counts_host[r];
         if (p < 0) return fail(TV_ERR_INVALID, "plan: negative prefix length for request %d", r);
@@ -192,6 +218,7 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
         const int npw = nodes_per_item(hpw, qpk);
         const int64_t groups = (num_kv_heads + hpw - 1) / hpw;
         const int64_t blocks = (t + npw - 1) / npw;
+        units += groups * blocks;
         total_cost += groups * blocks * cost_weight(hpw) * (static_cast<int64_t>(p) + t);
     }
     const int64_t target = std::max<int64_t>(kMinChunkKeys, total_cost / num_compute_units);
@@ -221,25 +248,40 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
             const int64_t p = prefix_lens_host[r];
             const int hpw = heads_per_group(node_counts_host[r], num_kv_heads, qpk);
             const int npw = nodes_per_item(hpw, qpk);
-            const int64_t units = static_cast<int64_t>((num_kv_heads + hpw - 1) / hpw) * ((node_counts_host[r] + npw - 1) / npw);
+            const int64_t per = static_cast<int64_t>((num_kv_heads + hpw - 1) / hpw) * ((node_counts_host[r] + npw - 1) / npw);
             const int64_t chunk = chunk_for(p, node_counts_host[r], hpw, tau);
-            n += units * (p > 0 ? (p + chunk - 1) / chunk : 1);
+            n += per * (p > 0 ? (p + chunk - 1) / chunk : 1);
         }
         return n;
     };
     int64_t tau = target;
-    if (chunk_keys == 0) {
-        const int64_t now = items_for(target);
-        const int64_t rounds = (now + num_compute_units - 1) / num_compute_units;
-        // Rounds already full: every smaller target that keeps the item count keeps every
-        // request's chunk count (each is non-increasing in the target), so the plan is this one.
-        if (now > num_compute_units && rounds <= kFillRounds && now < rounds * num_compute_units) {
-            int64_t lo = 1, hi = target;   // items_for(hi) fits `rounds` full rounds
+    const int64_t now = chunk_keys == 0 ? items_for(target) : 0;
+    if (chunk_keys == 0 && now <= kFillRounds * num_compute_units) {
+        // Smallest multiple of kTauStep whose item count is at most `cap`; 0 if an uncut batch has more.
+        auto fit = [&](int64_t cap) -> int64_t {
+            const int64_t most = total_cost / kTauStep + 1;   // uncut
+            int64_t lo = 1, hi = std::max<int64_t>(1, std::min(most, total_cost / cap / kTauStep));
+            while (items_for(hi * kTauStep) > cap) {
+                if (hi >= most) return 0;
+                lo = hi + 1;
+                hi = std::min(most, 2 * hi);
+            }
             while (lo < hi) {
                 const int64_t mid = lo + (hi - lo) / 2;
-                if (items_for(mid) <= rounds * num_compute_units) hi = mid; else lo = mid + 1;
+                if (items_for(mid * kTauStep) <= cap) hi = mid; else lo = mid + 1;
             }
-            tau = lo;
+            return lo * kTauStep;
+        };
+        const int64_t rounds = std::max<int64_t>(1, (now + num_compute_units - 1) / num_compute_units);
+        int64_t best = 0;
+        for (int64_t k = 1; k <= rounds; ++k) {
+            const int64_t cap = k == 1 ? one_round_items(total_cost, units, num_compute_units) : k * num_compute_units;
+            const int64_t t = fit(cap);
+            const int64_t span = k * (t + kRoundCost) + kSlotCost * cap;
+            if (t > 0 && (best == 0 || span < best)) {
+                best = span;
+                tau = t;
+            }
         }
     }
 

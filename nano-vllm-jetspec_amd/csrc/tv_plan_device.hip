@@ -64,6 +64,24 @@ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + 
 // planner uses the same weights.
 __device__ __forceinline__ int64_t cost_weight(int hpw) { return hpw == 2 ? 5 : 4; }
 
+// The host planner's choice of the chunk target (tv_plan.cpp gives the reasons and figures).
+constexpr int64_t kPartialCost = 8;
+constexpr int64_t kRoundCost = 1000;
+constexpr int64_t kSlotCost = 2;
+constexpr int64_t kTauStep = 128;
+
+__device__ __forceinline__ int64_t one_round_items(int64_t total_cost, int64_t units, int64_t compute_units) {
+    const int64_t x = total_cost / kPartialCost;
+    int64_t n = compute_units;
+    if (x < compute_units * compute_units) {
+        n = 0;
+        for (int64_t bit = int64_t{1} << 20; bit > 0; bit >>= 1) {   // integer square root
+            if ((n + bit) * (n + bit) <= x) n += bit;
+        }
+    }
+    return min(compute_units, max(n, units));
+}
+
 constexpr int kPlanWaves = kPlanThreads / 64;
 constexpr int kPer = kMaxSortItems / kPlanThreads;   // sorted positions per thread
 constexpr int kProbeWaves = 4;   // waves that probe chunk targets in the refit (one per SIMD)
@@ -218,7 +236,6 @@ plan_device_kernel(const PlanArgs a) {
     __shared__ int shape_flag;   // bit 0: some request has several node blocks; bit 1: one not a multiple of 8
     __shared__ int class_singles;   // single items of a cost-class plan
     __shared__ int32_t probe_fits[kPlanWaves];
-    __shared__ int64_t probe_val[kPlanWaves];
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -298,7 +315,7 @@ plan_device_kernel(const PlanArgs a) {
         }
         bool bad = false;
         int my_shapes = 0;
-        int64_t my_cost = 0;
+        int64_t my_cost = 0, my_units = 0;
         for (int r = t; r < R; r += kPlanThreads) {
             const int p = a.prefix_lens[r], n = a.node_counts[r];
             bad |= p < 0 || n < 1 || n > kMaxPlanNodes;
@@ -308,6 +325,7 @@ plan_device_kernel(const PlanArgs a) {
             const ReqShape s = req_shape(nc, KV, NW);
             req_bits[r] = static_cast<uint16_t>(s.NB | (s.hpw == 2 ? 0x8000 : 0));
             my_shapes |= (s.NB > 1 ? 1 : 0) | (s.NB > 1 && s.NB % kXcds ? 2 : 0);
+            my_units += static_cast<int64_t>(s.G) * s.NB;
             my_cost += static_cast<int64_t>(s.G) * s.NB * cost_weight(s.hpw) * (static_cast<int64_t>(pc) + nc);
         }
         if (!one_wave) __syncthreads();   // the flags are cleared before anyone sets them
@@ -316,6 +334,8 @@ plan_device_kernel(const PlanArgs a) {
         // The block sum's barriers also publish req_p, req_n, req_bits and the flags.
         const int64_t total_cost = one_wave ? wave_sum(my_cost)
                                             : block_sum(my_cost, (min(R, kPlanThreads) + 63) / 64, scan);
+        const int64_t units = one_wave ? wave_sum(my_units)
+                                       : block_sum(my_units, (min(R, kPlanThreads) + 63) / 64, scan);
         const int64_t target = max(static_cast<int64_t>(kMinChunkKeys), total_cost / a.compute_units);
 
         // 2. Chunking and per-request counts at chunk target tau (or the forced chunk length):
@@ -378,55 +398,92 @@ plan_device_kernel(const PlanArgs a) {
         };
         chunking(target);
 
-        // 2b. The host's refit of the chunk target when the items leave the last of at most
-        // kFillRounds rounds part-empty: the smallest target whose item count fits the same
-        // rounds, then the chunking again at it.  When the rounds are already full, every
-        // smaller target that keeps the item count keeps every request's chunk count (each is
-        // non-increasing in the target), so the plan stands.  The count falls as the target
-        // grows, so any search finds the host's bisection result: wave 0 alone bisects; the
-        // block has one wave per SIMD probe one target per round (a 5-way search, two
-        // barriers per round; more probing waves would share the SIMDs and make every round
-        // as much longer).
-        if (a.chunk_keys == 0) {
-            const int64_t now = tot[0];
-            const int64_t rounds = (now + a.compute_units - 1) / a.compute_units;
-            if (now > a.compute_units && rounds <= kFillRounds && now < rounds * a.compute_units) {
-                const int64_t limit = rounds * a.compute_units;
-                int64_t lo = 1, hi = target;   // items(hi) <= limit; the answer is in [lo, hi]
+        // 2b. The host's choice of the chunk target for at most kFillRounds rounds of items, then
+        // the chunking again at it.  The count falls as the target grows, so any search finds the
+        // host's result: wave 0 alone gallops and bisects; the block has one wave per SIMD probe
+        // one target each (a 5-way search, two barriers per step; more probing waves would share
+        // the SIMDs and make every step as much longer).
+        if (a.chunk_keys == 0 && tot[0] <= kFillRounds * a.compute_units) {
+            // Whether the items at v[k] * kTauStep fit `cap`, bit k, in every thread taking part.
+            auto count_at = [&](int64_t i) -> int64_t {
+                const int64_t q4 = i * kTauStep / 4, q5 = i * kTauStep / 5;
+                int64_t n = 0;
+                for (int r = lane; r < R; r += 64) n += request_items(r, q4, q5);
+                return wave_sum(n);
+            };
+            auto probe4 = [&](int64_t v0, int64_t v1, int64_t v2, int64_t v3, int64_t cap) -> int {
+                if (wave < kProbeWaves) {
+                    const int64_t v = wave == 0 ? v0 : wave == 1 ? v1 : wave == 2 ? v2 : v3;
+                    const int64_t n = count_at(v);
+                    if (lane == 0) probe_fits[wave] = n <= cap ? 1 : 0;
+                }
+                __syncthreads();
+                int bits = 0;
+#pragma unroll
+                for (int k = 0; k < kProbeWaves; ++k) bits |= probe_fits[k] << k;
+                __syncthreads();   // every thread has read probe_fits
+                return bits;
+            };
+            const int64_t most = total_cost / kTauStep + 1;   // uncut
+            auto fit = [&](int64_t cap) -> int64_t {
+                int64_t lo = 1, hi = max(int64_t{1}, min(most, total_cost / cap / kTauStep));
                 if (one_wave) {
+                    while (count_at(hi) > cap) {
+                        if (hi >= most) return 0;
+                        lo = hi + 1;
+                        hi = min(most, 2 * hi);
+                    }
                     while (lo < hi) {
                         const int64_t mid = lo + (hi - lo) / 2;
-                        const int64_t n = wave_sum(lane < R ? request_items(lane, mid / 4, mid / 5) : 0);
-                        if (n <= limit) hi = mid; else lo = mid + 1;
+                        if (count_at(mid) <= cap) hi = mid; else lo = mid + 1;
                     }
                 } else {
+                    for (;;) {
+                        const int64_t v1 = min(most, 2 * hi), v2 = min(most, 4 * hi), v3 = min(most, 8 * hi);
+                        const int bits = probe4(hi, v1, v2, v3, cap);   // fits from some bit on
+                        if (bits & 1) break;
+                        lo = hi + 1;
+                        hi = v1;
+                        if (bits & 2) break;
+                        lo = v1 + 1;
+                        hi = v2;
+                        if (bits & 4) break;
+                        lo = v2 + 1;
+                        hi = v3;
+                        if (bits & 8) break;
+                        if (v3 >= most) return 0;
+                        lo = v3 + 1;
+                        hi = min(most, 2 * v3);
+                    }
                     while (lo < hi) {
                         const int64_t span = hi - lo;
-                        if (wave < kProbeWaves) {
-                            const int64_t probe = lo + span * (wave + 1) / (kProbeWaves + 1);   // in [lo, hi)
-                            const int64_t q4 = probe / 4, q5 = probe / 5;
-                            int64_t n = 0;
-                            for (int r = lane; r < R; r += 64) n += request_items(r, q4, q5);
-                            n = wave_sum(n);
-                            if (lane == 0) {
-                                probe_fits[wave] = n <= limit ? 1 : 0;
-                                probe_val[wave] = probe;
-                            }
-                        }
-                        __syncthreads();
+                        const int64_t v0 = lo + span / 5, v1 = lo + span * 2 / 5, v2 = lo + span * 3 / 5,
+                                      v3 = lo + span * 4 / 5;   // in [lo, hi)
+                        const int bits = probe4(v0, v1, v2, v3, cap);
+                        const int64_t v[4] = {v0, v1, v2, v3};
                         int64_t new_lo = lo, new_hi = hi;
 #pragma unroll
-                        for (int k = 0; k < kProbeWaves; ++k) {
-                            const int64_t pk = probe_val[k];
-                            if (probe_fits[k]) new_hi = min(new_hi, pk); else new_lo = max(new_lo, pk + 1);
+                        for (int k = 0; k < 4; ++k) {
+                            if (bits >> k & 1) new_hi = min(new_hi, v[k]); else new_lo = max(new_lo, v[k] + 1);
                         }
-                        __syncthreads();   // every thread has read probe_fits
                         lo = new_lo;
                         hi = new_hi;
                     }
                 }
-                if (lo != target) chunking(lo);
+                return lo * kTauStep;
+            };
+            const int64_t rounds = max(int64_t{1}, (tot[0] + a.compute_units - 1) / a.compute_units);
+            int64_t best = 0, tau = target;
+            for (int64_t k = 1; k <= rounds; ++k) {
+                const int64_t cap = k == 1 ? one_round_items(total_cost, units, a.compute_units) : k * a.compute_units;
+                const int64_t found = fit(cap);
+                const int64_t span = k * (found + kRoundCost) + kSlotCost * cap;
+                if (found > 0 && (best == 0 || span < best)) {
+                    best = span;
+                    tau = found;
+                }
             }
+            if (tau != target) chunking(tau);
         }
         if (one_wave && lane < R) write_classes(lane);
     }
