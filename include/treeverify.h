@@ -249,6 +249,19 @@ int tv_truncate_accepted(const int32_t* paths, int32_t path_stride, const int32_
                          int32_t* limits, int64_t* emitted, int32_t* commit_paths,
                          int32_t* commit_offsets, int32_t* status, void* stream);
 
+/*
+ * tv_truncate_accepted with the EOS ids in host memory: at most TV_MAX_HOST_EOS of them (else
+ * TV_ERR_UNSUPPORTED), read before the call returns and passed in the kernel's arguments, so the
+ * cut waits for no upload.
+ */
+#define TV_MAX_HOST_EOS 8
+int tv_truncate_accepted_host_eos(const int32_t* paths, int32_t path_stride, const int32_t* lengths,
+                                  const int64_t* corrections, const void* token_ids, int32_t tokens_is_int64,
+                                  const int32_t* cu_seqlens, int32_t num_requests, const int32_t* budgets,
+                                  const uint8_t* ignore_eos, const int64_t* eos_token_ids_host, int32_t num_eos,
+                                  int32_t* limits, int64_t* emitted, int32_t* commit_paths,
+                                  int32_t* commit_offsets, int32_t* status, void* stream);
+
 /* ------------------------------------------------------------------------- */
 /* packed tree attention  (speculative/jetspec/paged_backend.py:240-306)      */
 /* ------------------------------------------------------------------------- */

@@ -289,11 +289,29 @@ namespace tv {
 namespace {
 constexpr int kTruncThreads = 1024;
 
+// The EOS ids: from device memory, or the caller's few host ids in the kernel's arguments.
+struct EosIds {
+    const int64_t* device;   // nullptr: held
+    int32_t count;
+    int64_t held[TV_MAX_HOST_EOS];
+};
+
+__device__ __forceinline__ bool is_eos(const EosIds& eos, int64_t value) {
+    bool hit = false;
+    if (eos.device) {
+        for (int32_t e = 0; e < eos.count; ++e) hit = hit || value == eos.device[e];
+    } else {
+#pragma unroll
+        for (int32_t e = 0; e < TV_MAX_HOST_EOS; ++e) hit = hit || (e < eos.count && value == eos.held[e]);
+    }
+    return hit;
+}
+
 __global__ void __launch_bounds__(kTruncThreads)
 truncate_accepted_kernel(const int32_t* __restrict__ paths, int32_t stride, const int32_t* __restrict__ lengths,
                          const int64_t* __restrict__ corrections, const void* __restrict__ tokens, int tokens64,
                          const int32_t* __restrict__ cu, int32_t num_requests, const int32_t* __restrict__ budgets,
-                         const uint8_t* __restrict__ ignore_eos, const int64_t* __restrict__ eos, int32_t num_eos,
+                         const uint8_t* __restrict__ ignore_eos, const EosIds eos,
                          int32_t* __restrict__ limits, int64_t* __restrict__ emitted,
                          int32_t* __restrict__ commit_paths, int32_t* __restrict__ commit_offsets, int32_t* status) {
     __shared__ int32_t scan[kTruncThreads];
@@ -323,9 +341,7 @@ truncate_accepted_kernel(const int32_t* __restrict__ paths, int32_t stride, cons
                 if (!ignore_eos[r]) {
                     for (int32_t j = 0; j < limit; ++j) {
                         const int64_t v = value(j);
-                        bool hit = false;
-                        for (int32_t e = 0; e < num_eos; ++e) hit = hit || v == eos[e];
-                        if (hit) {
+                        if (is_eos(eos, v)) {
                             limit = j + 1;
                             break;
                         }
@@ -370,7 +386,7 @@ truncate_teams_kernel(const int32_t* __restrict__ paths, int32_t stride, int32_t
                       const int32_t* __restrict__ lengths, const int64_t* __restrict__ corrections,
                       const void* __restrict__ tokens, int tokens64, const int32_t* __restrict__ cu,
                       int32_t num_requests, const int32_t* __restrict__ budgets,
-                      const uint8_t* __restrict__ ignore_eos, const int64_t* __restrict__ eos, int32_t num_eos,
+                      const uint8_t* __restrict__ ignore_eos, const EosIds eos,
                       int32_t* __restrict__ limits, int64_t* __restrict__ emitted,
                       int32_t* __restrict__ commit_paths, int32_t* __restrict__ commit_offsets, int32_t* status) {
     __shared__ int32_t pass_limits[2][64];   // by the pass's parity: one barrier a pass
@@ -406,9 +422,7 @@ truncate_teams_kernel(const int32_t* __restrict__ paths, int32_t stride, int32_t
                     value = tokens64 ? static_cast<const int64_t*>(tokens)[row]
                                      : static_cast<int64_t>(static_cast<const int32_t*>(tokens)[row]);
                 }
-                bool hit = false;
-                for (int32_t e = 0; e < num_eos; ++e) hit = hit || value == eos[e];
-                const uint64_t ends = __ballot(wanted && j < limit && hit) & members;
+                const uint64_t ends = __ballot(wanted && j < limit && is_eos(eos, value)) & members;
                 if (ends) limit = __builtin_ctzll(ends) - first + 1;
             }
             if (j == 0) limits[r] = limit;
@@ -434,15 +448,13 @@ truncate_teams_kernel(const int32_t* __restrict__ paths, int32_t stride, int32_t
 }  // namespace
 }  // namespace tv
 
-extern "C" int tv_truncate_accepted(const int32_t* paths, int32_t path_stride, const int32_t* lengths,
-                                    const int64_t* corrections, const void* token_ids, int32_t tokens_is_int64,
-                                    const int32_t* cu_seqlens, int32_t num_requests, const int32_t* budgets,
-                                    const uint8_t* ignore_eos, const int64_t* eos_token_ids, int32_t num_eos,
-                                    int32_t* limits, int64_t* emitted, int32_t* commit_paths,
-                                    int32_t* commit_offsets, int32_t* status, void* stream) {
-    using namespace tv;
-    clear_error();
-    if (num_requests < 0 || path_stride < 1 || num_eos < 0) {
+namespace tv {
+namespace {
+int truncate_accepted(const int32_t* paths, int32_t path_stride, const int32_t* lengths, const int64_t* corrections,
+                      const void* token_ids, int32_t tokens_is_int64, const int32_t* cu_seqlens, int32_t num_requests,
+                      const int32_t* budgets, const uint8_t* ignore_eos, const EosIds& eos, int32_t* limits,
+                      int64_t* emitted, int32_t* commit_paths, int32_t* commit_offsets, int32_t* status, void* stream) {
+    if (num_requests < 0 || path_stride < 1 || eos.count < 0) {
         return fail(TV_ERR_INVALID, "truncate_accepted: invalid request count, path stride or EOS count");
     }
     if (num_requests == 0) return TV_OK;
@@ -450,7 +462,7 @@ extern "C" int tv_truncate_accepted(const int32_t* paths, int32_t path_stride, c
         return fail(TV_ERR_UNSUPPORTED, "truncate_accepted: too many path entries");
     }
     if (!paths || !lengths || !corrections || !token_ids || !cu_seqlens || !budgets || !ignore_eos || !limits ||
-        !emitted || !commit_paths || !commit_offsets || (num_eos > 0 && !eos_token_ids)) {
+        !emitted || !commit_paths || !commit_offsets) {
         return fail(TV_ERR_INVALID, "truncate_accepted: null pointer");
     }
     // A team of 16 to 64 lanes per request up to 256 requests: a pass of 64 requests adds 2.5 us
@@ -462,13 +474,54 @@ extern "C" int tv_truncate_accepted(const int32_t* paths, int32_t path_stride, c
         static_assert(kTeamMinLanes == 1 << 4 && kTruncThreads / kTeamMinLanes <= 64, "one lane per team in the scan");
         hipLaunchKernelGGL(truncate_teams_kernel, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths,
                            path_stride, shift, lengths, corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0,
-                           cu_seqlens, num_requests, budgets, ignore_eos, eos_token_ids, num_eos, limits, emitted,
-                           commit_paths, commit_offsets, status);
+                           cu_seqlens, num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths,
+                           commit_offsets, status);
         return check_launch("truncate_accepted");
     }
     hipLaunchKernelGGL(truncate_accepted_kernel, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths,
                        path_stride, lengths, corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0, cu_seqlens,
-                       num_requests, budgets, ignore_eos, eos_token_ids, num_eos, limits, emitted, commit_paths,
-                       commit_offsets, status);
+                       num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths, commit_offsets, status);
     return check_launch("truncate_accepted");
+}
+}  // namespace
+}  // namespace tv
+
+extern "C" int tv_truncate_accepted(const int32_t* paths, int32_t path_stride, const int32_t* lengths,
+                                    const int64_t* corrections, const void* token_ids, int32_t tokens_is_int64,
+                                    const int32_t* cu_seqlens, int32_t num_requests, const int32_t* budgets,
+                                    const uint8_t* ignore_eos, const int64_t* eos_token_ids, int32_t num_eos,
+                                    int32_t* limits, int64_t* emitted, int32_t* commit_paths,
+                                    int32_t* commit_offsets, int32_t* status, void* stream) {
+    using namespace tv;
+    clear_error();
+    if (num_eos > 0 && num_requests > 0 && !eos_token_ids) {
+        return fail(TV_ERR_INVALID, "truncate_accepted: null pointer");
+    }
+    EosIds eos = {};
+    eos.device = eos_token_ids;
+    eos.count = num_eos;
+    return truncate_accepted(paths, path_stride, lengths, corrections, token_ids, tokens_is_int64, cu_seqlens,
+                             num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths, commit_offsets,
+                             status, stream);
+}
+
+extern "C" int tv_truncate_accepted_host_eos(const int32_t* paths, int32_t path_stride, const int32_t* lengths,
+                                             const int64_t* corrections, const void* token_ids,
+                                             int32_t tokens_is_int64, const int32_t* cu_seqlens, int32_t num_requests,
+                                             const int32_t* budgets, const uint8_t* ignore_eos,
+                                             const int64_t* eos_token_ids_host, int32_t num_eos, int32_t* limits,
+                                             int64_t* emitted, int32_t* commit_paths, int32_t* commit_offsets,
+                                             int32_t* status, void* stream) {
+    using namespace tv;
+    clear_error();
+    if (num_eos > TV_MAX_HOST_EOS) {
+        return fail(TV_ERR_UNSUPPORTED, "truncate_accepted: %d host EOS ids, at most %d", num_eos, TV_MAX_HOST_EOS);
+    }
+    if (num_eos > 0 && !eos_token_ids_host) return fail(TV_ERR_INVALID, "truncate_accepted: null pointer");
+    EosIds eos = {};
+    eos.count = num_eos;
+    for (int32_t e = 0; e < num_eos; ++e) eos.held[e] = eos_token_ids_host[e];
+    return truncate_accepted(paths, path_stride, lengths, corrections, token_ids, tokens_is_int64, cu_seqlens,
+                             num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths, commit_offsets,
+                             status, stream);
 }

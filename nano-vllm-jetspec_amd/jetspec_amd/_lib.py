@@ -32,6 +32,8 @@ TV_STATUS_BAD_DEPTH = 16
 TV_STATUS_BAD_BIAS = 32
 TV_STATUS_STALE_PLAN = 64
 
+TV_MAX_HOST_EOS = 8
+
 # Every extern "C" symbol of include/treeverify.h.
 EXPORTED_SYMBOLS = (
     "tv_abi_version",
@@ -42,6 +44,7 @@ EXPORTED_SYMBOLS = (
     "tv_copy_accepted_kv",
     "tv_commit_slots",
     "tv_truncate_accepted",
+    "tv_truncate_accepted_host_eos",
     "tv_tree_attention_plan",
     "tv_tree_attention_plan_slots",
     "tv_pack_ancestor_words",
@@ -207,6 +210,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tv_truncate_accepted.argtypes = [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_int32,
                                          c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p,
                                          c_void_p, c_void_p, c_void_p]
+    lib.tv_truncate_accepted_host_eos.restype = c_int32
+    lib.tv_truncate_accepted_host_eos.argtypes = [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
+                                                  c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
+                                                  c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
     lib.tv_tree_attention_plan.restype = c_int32
     lib.tv_tree_attention_plan.argtypes = [POINTER(c_int32), POINTER(c_int32), c_int32, c_int32, c_int32,
                                            c_int32, c_int32, c_int32, POINTER(c_int32), POINTER(c_int32),

@@ -48,7 +48,7 @@ def test_walk_and_cut_equal_the_oracle(max_depth, sizes, index_dtype):
 
     budgets = torch.tensor(rng.integers(1, max_depth + 4, size=len(sizes)), dtype=torch.int32)
     ignore = torch.tensor(rng.random(len(sizes)) < 0.3)
-    for count in (0, 1, 8, 9):
+    for count in (0, 1, 8, 9):   # up to 8 ids go with the launch, more are uploaded
         eos = {int(x) for x in rng.choice(VOCAB, size=count, replace=False)}
         limits, emitted, commit_paths, commit_offsets = truncate_accepted(
             paths, lengths, corrections, packed[0], cu, budgets.to(DEV), ignore.to(DEV), eos)
