@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import oracle
-from jetspec_amd import accept_batch_device, read_and_clear_status, truncate_accepted, workloads
+from jetspec_amd import accept_batch_device, greedy_argmax, read_and_clear_status, truncate_accepted, workloads
 from test_accept_gpu import DEV, expected_cuts, random_batch
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +82,24 @@ def test_bad_requests_beside_good_ones():
     assert commit_offsets.tolist() == np.concatenate([[0], np.cumsum(limits.tolist())]).tolist()
     assert commit_paths[:int(commit_offsets[-1])].tolist() == list(range(6)) * (requests - len(bad))
     assert read_and_clear_status(DEV) == 4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [1, 3, 7, 8, 9, 15, 2055, 50257])
+def test_argmax_of_rows_off_the_vector_boundary(dtype, vocab):
+    """Rows that start at every element offset from 16 bytes: the maximum, a tie and a NaN at the
+    first element, around the first vector unit and at the end, as torch.argmax has them."""
+    backing = torch.randn(16, vocab + 9, generator=torch.Generator(device=DEV).manual_seed(vocab), device=DEV).to(dtype)
+    marks = sorted({m for m in (0, 1, 2, 3, 4, 5, 6, 7, 8, 9, vocab // 2, vocab - 2, vocab - 1) if 0 <= m < vocab})
+    for start in range(9):
+        rows = backing[:, start:start + vocab]
+        for mark in marks:
+            case = rows.clone()
+            case[0, mark] = 50.0
+            case[1, mark] = case[1, marks[-1]] = 50.0
+            case[2, mark] = float("nan")
+            case[3, mark], case[3, marks[0]] = float("nan"), float("inf")
+            case[4] = float("-inf")
+            rows_at = torch.empty_like(backing)[:, start:start + vocab]
+            rows_at.copy_(case)
+            assert torch.equal(greedy_argmax(rows_at), rows_at.argmax(-1)), (start, mark)
