@@ -43,7 +43,10 @@ constexpr int64_t kFillRounds = 4;  // item rounds the chunk target is chosen fo
 // 496 items in two rounds 64.5 us, 244 in one 49.1; a one-head shard of 32 requests of
 // 1.1k-8.1k keys: 499 items 75.8 us, 227 items 53.9; 8 requests of 545-1603 keys and 32 nodes:
 // 236 items 29.9 us, 160 items 27.9.
-constexpr int64_t kPartialCost = 8;
+// kPartialCost of 3, 5 and 8, us: 8 requests of 1390-3225 keys on 2 KV heads 30.5, 29.0, 30.5
+// (204, 156, 138 items); 4 requests of 500-2000 keys on one 23.7, 21.6, 23.0; 16 of 2-8k keys on
+// one 30.9, 30.9, 31.8; 8 of 256-2048 keys on 8 29.2, 28.0, 28.5.
+constexpr int64_t kPartialCost = 5;
 constexpr int64_t kRoundCost = 1000;
 constexpr int64_t kSlotCost = 2;
 constexpr int64_t kTauStep = 128;   // 32 keys of a one-head item

@@ -65,7 +65,7 @@ __device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + 
 __device__ __forceinline__ int64_t cost_weight(int hpw) { return hpw == 2 ? 5 : 4; }
 
 // The host planner's choice of the chunk target (tv_plan.cpp gives the reasons and figures).
-constexpr int64_t kPartialCost = 8;
+constexpr int64_t kPartialCost = 5;
 constexpr int64_t kRoundCost = 1000;
 constexpr int64_t kSlotCost = 2;
 constexpr int64_t kTauStep = 128;
