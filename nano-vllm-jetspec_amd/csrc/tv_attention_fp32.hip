@@ -78,7 +78,7 @@ struct Fp32Params {
     int32_t groups;       // query heads per KV head
     int32_t head_dim;
     int32_t block_size;
-    float scale;          // softmax scale * log2(e): scores are kept in log2 units
+    float scale;          // softmax scale * log2(e) / 2: scores are kept in kUnit
     int32_t splits;       // chunks a row block's keys may be cut into (grid y)
     int32_t slots;        // workgroups the chip runs at a time
     int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
@@ -117,7 +117,13 @@ constexpr int64_t kCutRows = 4096;  // partial row blocks a workspace holds at m
 // Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
 // rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
 constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
-constexpr float kLog2eF = 1.4426950408889634f;
+// Scores and maxima are kept in units of two octaves (natural units * log2(e) / 2): the factor is
+// below 1, so that the most negative bias a mask can hold stays a finite score (in log2 units
+// torch.finfo(float32).min would become -inf and a row that sees nothing else a NaN).
+constexpr float kUnit = 1.4426950408889634f / 2;
+// A maximum beyond this is subtracted before the factor of two, which would overflow.
+constexpr float kHugeMax = 1e38f;
+__device__ __forceinline__ float exp2_units(float x) { return __builtin_amdgcn_exp2f(2.f * x); }
 
 // The launch numbers the row blocks of request r from start(r) = floor(cu[r] * G / 32) + r on:
 // the ranges are disjoint and increasing (start(r + 1) - start(r) >= ceil(T_r * G / 32)), so a
@@ -324,10 +330,10 @@ struct Op<float> {
     static constexpr float kShift = 0.f;
 };
 
-// A score more than this far above a row's reference maximum (log2 units) raises the
+// A score more than this far above a row's reference maximum (2^8 in probability) raises the
 // maximum; below it probabilities stay <= 2^8, which fp32 holds with its full relative
 // precision, so the result is the same online softmax with rare rescales.
-constexpr float kRaiseMargin = 8.f;
+constexpr float kRaiseMargin = 4.f;
 
 // T: operand type; DIM: the head size, or (EXACT false) an upper bound of it in {64, 128, 256,
 // 512} with loads and products past p.head_dim left out, and element loads where the rows do not
@@ -620,7 +626,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
         __builtin_amdgcn_sched_barrier(0);
         // Softmax of the 16 keys this lane holds (key 8 * (r / 4) + 4 * g + r % 4).
         const bool masked = here != ~0u || t0 + kTile > P;
-        const float mul = masked ? 1.f : cs;   // masked tiles hold finished scores, the others K.Q
+        float mul = masked ? 1.f : cs;   // masked tiles hold finished scores, the others K.Q
         float mx = -INFINITY;
         if (masked) {
 #pragma unroll
@@ -631,7 +637,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
                 if (visible && pos >= P) {
                     const float bias = bias_row[pos - P];
                     visible = bias != -INFINITY;
-                    x = fmaf(bias, kLog2eF, x);
+                    x = fmaf(bias, kUnit, x);
                 }
                 s[r] = visible ? x : -INFINITY;
                 mx = fmaxf(mx, s[r]);
@@ -644,14 +650,22 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
             // Both halves of a row decide on the whole row; rows that do not ask keep their maximum.
             const float row_max = fmaxf(mx, __shfl_xor(mx, 32));
             if (row_max > m + kRaiseMargin) {
-                const float alpha = __builtin_amdgcn_exp2f(m - row_max);   // 0 while m is -inf
+                const float alpha = exp2_units(m - row_max);   // 0 while m is -inf
                 l *= alpha;
 #pragma unroll
                 for (int n = 0; n < NB; ++n) acc[n] *= alpha;
                 m = row_max;
             }
         }
-        const float ref = m == -INFINITY ? 0.f : Op<T>::kShift - m;   // a score of -inf gives 0, whatever m
+        float ref = m == -INFINITY ? 0.f : Op<T>::kShift - 2.f * m;   // a score of -inf gives 0, whatever m
+        mul *= 2.f;
+        if (__any(fabsf(m) > kHugeMax && fabsf(m) < INFINITY)) {   // rows of lowest-value biases
+            const float top = m == -INFINITY ? 0.f : m;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = 2.f * (s[r] * (0.5f * mul) - top);
+            mul = 1.f;
+            ref = Op<T>::kShift;
+        }
         float l0 = 0.f, l1 = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
@@ -721,7 +735,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
     float row_m = ml_lds[0][c].x;
 #pragma unroll
     for (int w = 1; w < kWaves; ++w) row_m = fmaxf(row_m, ml_lds[w][c].x);
-    const float scale_w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - row_m);
+    const float scale_w = m == -INFINITY ? 0.f : exp2_units(m - row_m);
     float* o_lds = reinterpret_cast<float*>(smem);
     // acc block 2j + i, register r of half g: dim 64j + 2 * (8 * (r / 4) + 4 * g + r % 4) + i.
     auto o_at = [&](int buf, int j, int r) __attribute__((always_inline)) -> f32x2* {
@@ -765,7 +779,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             const float2 x = ml_lds[w][tid];
-            sum += x.x == -INFINITY ? 0.f : x.y * __builtin_amdgcn_exp2f(x.x - row_m);
+            sum += x.x == -INFINITY ? 0.f : x.y * exp2_units(x.x - row_m);
         }
         p.ws_ml[part + tid] = make_float2(row_m, sum);   // tid < 32: lane tid holds row tid's maximum
     }
@@ -779,7 +793,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) {
                 const float2 x = ml_lds[w][rr];
-                sum += x.x == -INFINITY ? 0.f : x.y * __builtin_amdgcn_exp2f(x.x - top);
+                sum += x.x == -INFINITY ? 0.f : x.y * exp2_units(x.x - top);
             }
             inv = 1.f / sum;
             const int node = (b.row0 + rr) / G, head = kvh * G + (b.row0 + rr) % G;
@@ -858,7 +872,7 @@ merge_fp32_kernel(const Fp32Params p) {
     float top = ml.x;
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
-    const float w = ml.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml.x - top);
+    const float w = ml.x == -INFINITY ? 0.f : exp2_units(ml.x - top);
     float sum = ml.y * w;
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
@@ -1034,7 +1048,7 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
     p.groups = a->num_q_heads / a->num_kv_heads;
     p.head_dim = a->head_dim;
     p.block_size = a->block_size;
-    p.scale = a->scale * kLog2eF;
+    p.scale = a->scale * kUnit;
     p.status = a->status;
     p.kv_heads = a->num_kv_heads;
     p.splits = 1;
