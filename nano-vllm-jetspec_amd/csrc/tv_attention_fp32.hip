@@ -26,9 +26,9 @@
 //     step v of V^T.P^T is the key that S^T register v of half g holds, so the
 //     probabilities feed the product from the registers the scores were computed in.
 //   16-bit operands: v_mfma_f32_32x32x16; the fp32 probability is split into three terms of
-//     the operand type (its rounding, the rounding of the remainder, and that of the rest:
-//     24 bits in bf16, 33 in f16), one product each, so it enters the sum with at least
-//     fp32's precision.
+//     the operand type (its rounding, the rounding of the remainder, and that of the rest),
+//     one product each: all 24 bits of it in bf16; in f16 to 2^-39 of the row's reference
+//     (Op<_Float16>), which is below what fp32 sums of it keep.
 //
 // What bounds it.  f32: the matrix core, 8192 cycles a tile and wave (a wave's tile takes 10.7 us
 // with two waves a SIMD, 7 us at the core's rate), and the uneven lengths of the workgroups.
@@ -314,6 +314,7 @@ struct Op<__bf16> {
     }
     // log2 of the factor the probabilities carry (it cancels against the row sum).
     static constexpr float kShift = 0.f;
+    static constexpr float kMargin = 4.f;
 };
 template <>
 struct Op<_Float16> {
@@ -321,19 +322,22 @@ struct Op<_Float16> {
     static __device__ __forceinline__ f32x16 mfma(vec a, vec b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
-    // Probabilities up to 2^8 become at most 2^15: the three f16 terms of one then reach down
-    // to 2^-31 of a probability of 1 instead of f16's 2^-24.
-    static constexpr float kShift = 7.f;
+    // The three terms end at f16's smallest step, 2^-24, so probabilities are scaled up to it as
+    // far as f16's range allows: at most 2 before the maximum is raised, 2^15 with the factor.  One
+    // is then held to 2^-39 of the row's reference, all 24 bits down to 2^-15 of it, and even 2^15
+    // keys rounded the same way shift the sum by no more than fp32's own rounding of it.
+    static constexpr float kShift = 14.f;
+    static constexpr float kMargin = 0.5f;
 };
 template <>
 struct Op<float> {
     static constexpr float kShift = 0.f;
+    static constexpr float kMargin = 4.f;
 };
 
-// A score more than this far above a row's reference maximum (2^8 in probability) raises the
-// maximum; below it probabilities stay <= 2^8, which fp32 holds with its full relative
+// A score more than Op::kMargin (4: 2^8 in probability) above a row's reference maximum raises
+// the maximum; below it probabilities stay <= 2^8, which fp32 holds with its full relative
 // precision, so the result is the same online softmax with rare rescales.
-constexpr float kRaiseMargin = 4.f;
 
 // T: operand type; DIM: the head size, or (EXACT false) an upper bound of it in {64, 128, 256,
 // 512} with loads and products past p.head_dim left out, and element loads where the rows do not
@@ -646,10 +650,10 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r] * cs);
         }
-        if (__any(mx > m + kRaiseMargin)) {   // rare after the first tile
+        if (__any(mx > m + Op<T>::kMargin)) {   // rare after the first tile
             // Both halves of a row decide on the whole row; rows that do not ask keep their maximum.
             const float row_max = fmaxf(mx, __shfl_xor(mx, 32));
-            if (row_max > m + kRaiseMargin) {
+            if (row_max > m + Op<T>::kMargin) {
                 const float alpha = exp2_units(m - row_max);   // 0 while m is -inf
                 l *= alpha;
 #pragma unroll

@@ -54,3 +54,29 @@ def test_lowest_value_masks(prefix, nodes, dtype):
     print(f"[lowest P{prefix} n{nodes} {dtype}] max-abs {error:.2e}", flush=True)
     assert error <= 1e-5
     assert read_and_clear_status(DEV) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("octaves", [10, 14, 16, 18, 20])
+def test_small_probabilities_beside_a_dominant_one(octaves, dtype):
+    """One key at the maximum with V = 0 and 8191 keys of one lower score with V = 1: the output is the
+    sum of the small probabilities alone, all rounded alike, so its relative error is theirs.
+    Bound: 2^-19 is the rounding of one held to 2^-39 of the reference at 2^-20 of it; the fp32
+    score (below 16 in log2 units, 2^-20 there), exponential and sums add at most as much."""
+    q, k, v, meta, *_ = make_case((8150,), (42,), kv_heads=1, groups=3, head_dim=96, dtype=dtype, seed=3)
+    k.zero_(), v.fill_(1.0), q.zero_()
+    q[..., 0] = 1.0
+    top = meta.block_tables_host[0][0]   # position 3
+    k[top, 3, 0, 0], v[top, 3] = 1.0, 0.0
+    worst = 0.0
+    for step in range(8):   # probabilities over one octave: the rounding of some is near the worst
+        scale = (octaves + step / 8) * float(np.log(2.0))
+        out = packed_tree_attention(q, k, v, meta, scale, 3, output_dtype=torch.float32)
+        keys = (meta.prefix_lengths[0] + 1 + torch.tensor(
+            [int((meta.qq_bias[i * 42:i * 42 + 42] == 0).sum()) - 1 for i in range(42)])).double()
+        small = (keys - 1) * np.exp(-np.float64(np.float32(scale)))
+        expect = (small / (1.0 + small)).view(-1, 1, 1)
+        worst = max(worst, ((out.cpu().double() - expect) / expect).abs().max().item())
+    print(f"[octaves {octaves} {dtype}] relative {worst:.2e}", flush=True)
+    assert worst <= 2.0 ** -18
+    assert read_and_clear_status(DEV) == 0
