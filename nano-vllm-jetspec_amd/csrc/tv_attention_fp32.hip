@@ -121,8 +121,7 @@ constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
 // below 1, so that the most negative bias a mask can hold stays a finite score (in log2 units
 // torch.finfo(float32).min would become -inf and a row that sees nothing else a NaN).
 constexpr float kUnit = 1.4426950408889634f / 2;
-// A maximum beyond this is subtracted before the factor of two, which would overflow.
-constexpr float kHugeMax = 1e38f;
+// The maximum is subtracted before the factor of two, which would overflow.
 __device__ __forceinline__ float exp2_units(float x) { return __builtin_amdgcn_exp2f(2.f * x); }
 
 // The launch numbers the row blocks of request r from start(r) = floor(cu[r] * G / 32) + r on:
@@ -630,7 +629,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
         __builtin_amdgcn_sched_barrier(0);
         // Softmax of the 16 keys this lane holds (key 8 * (r / 4) + 4 * g + r % 4).
         const bool masked = here != ~0u || t0 + kTile > P;
-        float mul = masked ? 1.f : cs;   // masked tiles hold finished scores, the others K.Q
+        const float mul = masked ? 1.f : cs;   // masked tiles hold finished scores, the others K.Q
         float mx = -INFINITY;
         if (masked) {
 #pragma unroll
@@ -661,19 +660,11 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
                 m = row_max;
             }
         }
-        float ref = m == -INFINITY ? 0.f : Op<T>::kShift - 2.f * m;   // a score of -inf gives 0, whatever m
-        mul *= 2.f;
-        if (__any(fabsf(m) > kHugeMax && fabsf(m) < INFINITY)) {   // rows of lowest-value biases
-            const float top = m == -INFINITY ? 0.f : m;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 2.f * (s[r] * (0.5f * mul) - top);
-            mul = 1.f;
-            ref = Op<T>::kShift;
-        }
+        const float ref = m == -INFINITY ? 0.f : -m;   // a score of -inf gives 0, whatever m
         float l0 = 0.f, l1 = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float pr = __builtin_amdgcn_exp2f(fmaf(s[r], mul, ref));
+            const float pr = __builtin_amdgcn_exp2f(fmaf(fmaf(s[r], mul, ref), 2.f, Op<T>::kShift));
             s[r] = pr;
             if (r & 1) l1 += pr; else l0 += pr;
         }
