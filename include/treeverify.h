@@ -565,6 +565,15 @@ int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries, int32_t nu
                                                int32_t num_kv_heads, int32_t head_dim);
 int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* args, void* workspace,
                                  int64_t workspace_bytes, void* stream);
+/*
+ * How a launch with a workspace cuts a batch of these lengths (host arrays): the longest chunk of
+ * a row block's keys (0: batches of this shape are never cut) and the workgroups that have work.
+ * The kernel takes the same decision from the live lengths.
+ */
+int tv_tree_attention_fp32_chunk_keys(const int32_t* prefix_lens_host, const int32_t* node_counts_host,
+                                      int32_t num_requests, int32_t num_q_heads, int32_t num_kv_heads,
+                                      int32_t head_dim, int32_t in_dtype, int32_t* chunk_keys,
+                                      int32_t* workgroups);
 /* sizeof(tv_tree_attention_fp32_args) as compiled, for binding layout checks. */
 int64_t tv_sizeof_tree_attention_fp32_args(void);
 

@@ -79,7 +79,7 @@ struct Fp32Params {
     int32_t head_dim;
     int32_t block_size;
     float scale;          // softmax scale * log2(e) / 2: scores are kept in kUnit
-    int32_t splits;       // chunks a row block's keys may be cut into (grid y)
+    int32_t splits;       // chunks a row block's keys may be cut into
     int32_t slots;        // workgroups the chip runs at a time
     int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
     int32_t kv_heads;
@@ -114,6 +114,7 @@ constexpr int kThreadsFp32 = kWave * kWaves;
 constexpr int kMaxSplits = 16;
 constexpr int kCus = 256;           // compute units of an MI355X
 constexpr int64_t kCutRows = 4096;  // partial row blocks a workspace holds at most
+constexpr int kCutRequests = kWave; // requests of a batch that is cut at most (one lane each)
 // Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
 // rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
 constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
@@ -221,22 +222,44 @@ __device__ __forceinline__ int wave_max(int x) {   // of non-negative values
 }
 
 // The cut of a batch whose keys are split (p.splits > 1, at most kCutRequests requests), the
-// same in every wave that computes it: chunks of at most `target` tiles, so that the workgroups
-// fill the chip once (p.slots of them run at a time: a part-filled second round would double the
-// launch), or as many times as the row blocks alone do.  Lane l holds request l.
-constexpr int kCutRequests = kWave;
+// same in every wave that computes it: chunks of at most `target` tiles (cut_target), so that
+// the workgroups fill the chip once (p.slots of them run at a time: a part-filled second round
+// would double the launch), or as many times as the row blocks alone do.  Lane l holds request l.
 struct Cut {
     int cu, nodes, prefix;   // the request's live metadata
     int blocks, tiles;       // its row blocks and the tiles of its keys
     int target;
 };
 
-__device__ __forceinline__ int chunks_of(int tiles, int target) {
+__host__ __device__ __forceinline__ int chunks_of(int tiles, int target) {
     return static_cast<int>((static_cast<uint32_t>(tiles) + target - 1) / static_cast<uint32_t>(target));
 }
 // Tiles of one of `parts` even chunks, in whole turns of the waves.
 __device__ __forceinline__ int chunk_tiles(int tiles, int parts) {
     return ((tiles + parts - 1) / parts + kWaves - 1) / kWaves * kWaves;
+}
+
+// Shortest chunk, in whole turns of the waves, whose workgroups fit `limit`: count(target) is
+// their number, which falls as the target grows and fits for an uncut batch.  The shortest is
+// the most even one.  `work` block-tiles over `limit` workgroups are a share no target goes
+// below, and the answer is mostly that share or little above it: every wave of the launch
+// searches upwards from there, about four counts.
+template <class Count>
+__host__ __device__ __forceinline__ int cut_target(int longest, int splits, int min_chunk, float work, int limit,
+                                                   Count count) {
+    const int even = static_cast<int>(fminf(work / limit, 1e9f));
+    const int floor = max(max(min_chunk, even), (longest + splits - 1) / splits);
+    const int most = (longest + kWaves - 1) / kWaves;   // uncut
+    int lo = (floor + kWaves - 1) / kWaves, hi = lo;
+    for (int step = 1; hi < most && count(hi * kWaves) > limit; step *= 2) {
+        lo = hi + 1;
+        hi = min(most, hi + step);
+    }
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (count(mid * kWaves) <= limit) hi = mid; else lo = mid + 1;
+    }
+    return lo * kWaves;
 }
 
 __device__ __forceinline__ Cut plan_cut(const Fp32Params& p) {
@@ -257,16 +280,9 @@ __device__ __forceinline__ Cut plan_cut(const Fp32Params& p) {
     const int longest = wave_max(cut.tiles);
     const int slots = p.slots * max(1, (units + p.slots - 1) / p.slots);
     const float work = wave_total(static_cast<float>(cut.blocks) * static_cast<float>(cut.tiles)) * p.kv_heads;
-    const int even = static_cast<int>(fminf(work / slots, 1e9f));
-    int target = max(max(even, p.min_chunk), (longest + p.splits - 1) / p.splits);
-    target = (target + kWaves - 1) / kWaves * kWaves;
-    // Last chunks are short, so the even share makes a few workgroups too many: longer chunks
-    // until they fit (each step is an eighth; 16 of them are an uncut batch's length).
-    for (int i = 0; i < 16 && target < longest; ++i) {
-        if (wave_total(cut.blocks * chunks_of(cut.tiles, target)) * p.kv_heads <= slots) break;
-        target += max(kWaves, target / 8 / kWaves * kWaves);
-    }
-    cut.target = target;
+    cut.target = cut_target(longest, p.splits, p.min_chunk, work, slots, [&](int target) {
+        return wave_total(cut.blocks * chunks_of(cut.tiles, target)) * p.kv_heads;
+    });
     return cut;
 }
 
@@ -900,6 +916,10 @@ int split_count(int64_t total_queries, int64_t num_requests, int64_t groups, int
     if (num_requests > kCutRequests) return 1;
     return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMaxSplits, kCutRows / units)));
 }
+int64_t blocks_of(int64_t nodes, int64_t groups) { return (nodes * groups + kBlockRows - 1) / kBlockRows; }
+// Workgroups the chip runs at a time (the kernel's launch bounds) and the shortest chunk.
+int chip_slots(int32_t head_dim) { return head_dim <= 128 ? 2 * kCus : kCus; }
+int min_chunk_tiles(int32_t in_dtype) { return in_dtype == TV_F32 ? kMinChunk32 : kMinChunk16; }
 int64_t partial_bytes(int64_t units, int splits, int32_t head_dim) {
     return units * splits * kBlockRows * (static_cast<int64_t>(head_dim) * 4 + static_cast<int64_t>(sizeof(float2)));
 }
@@ -969,6 +989,54 @@ extern "C" int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries,
     const int splits = split_count(total_queries, num_requests, groups, num_kv_heads);
     if (splits == 1) return 0;
     return partial_bytes(row_groups(total_queries, num_requests, groups) * num_kv_heads, splits, head_dim);
+}
+
+extern "C" int tv_tree_attention_fp32_chunk_keys(const int32_t* prefix_lens_host, const int32_t* node_counts_host,
+                                                 int32_t num_requests, int32_t num_q_heads, int32_t num_kv_heads,
+                                                 int32_t head_dim, int32_t in_dtype, int32_t* chunk_keys,
+                                                 int32_t* workgroups) {
+    clear_error();
+    if (!prefix_lens_host || !node_counts_host || !chunk_keys || !workgroups) {
+        return fail(TV_ERR_INVALID, "tree_attention_fp32_chunk_keys: null argument");
+    }
+    if (num_requests < 1 || num_kv_heads < 1 || num_q_heads < num_kv_heads || num_q_heads % num_kv_heads ||
+        head_dim < 1 || !valid_dtype(in_dtype)) {
+        return fail(TV_ERR_INVALID, "tree_attention_fp32_chunk_keys: invalid geometry");
+    }
+    const int64_t groups = num_q_heads / num_kv_heads;
+    int64_t queries = 0, units = 0, longest = 0;
+    double work = 0;
+    for (int32_t r = 0; r < num_requests; ++r) {
+        const int64_t keys = static_cast<int64_t>(prefix_lens_host[r]) + node_counts_host[r];
+        if (prefix_lens_host[r] < 0 || node_counts_host[r] < 0 || keys > INT32_MAX - kTile) {
+            return fail(TV_ERR_INVALID, "tree_attention_fp32_chunk_keys: invalid lengths of request %d", r);
+        }
+        queries += node_counts_host[r];
+        if (node_counts_host[r] == 0) continue;
+        units += blocks_of(node_counts_host[r], groups) * num_kv_heads;
+        longest = std::max(longest, (keys + kTile - 1) / kTile);
+        work += static_cast<double>(blocks_of(node_counts_host[r], groups) * num_kv_heads) * ((keys + kTile - 1) / kTile);
+    }
+    *chunk_keys = 0;
+    *workgroups = static_cast<int32_t>(units);
+    const int splits = split_count(queries, num_requests, groups, num_kv_heads);
+    if (splits == 1 || longest == 0) return TV_OK;
+    auto count = [&](int target) {
+        int64_t n = 0;
+        for (int32_t r = 0; r < num_requests; ++r) {
+            if (node_counts_host[r] == 0) continue;
+            const int tiles = static_cast<int>((static_cast<int64_t>(prefix_lens_host[r]) + node_counts_host[r] + kTile - 1) / kTile);
+            n += blocks_of(node_counts_host[r], groups) * chunks_of(tiles, target);
+        }
+        return static_cast<int>(n * num_kv_heads);
+    };
+    const int slots = chip_slots(head_dim);
+    const int limit = static_cast<int>(slots * std::max<int64_t>(1, (units + slots - 1) / slots));
+    const int target = cut_target(static_cast<int>(longest), splits, min_chunk_tiles(in_dtype),
+                                  static_cast<float>(work), limit, count);
+    *chunk_keys = target * kTile;
+    *workgroups = count(target);
+    return TV_OK;
 }
 
 extern "C" int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* a, void* stream) {
@@ -1058,8 +1126,8 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
                             (long long)workspace_bytes, (long long)partial_bytes(units, splits, a->head_dim));
             }
             p.splits = splits;
-            p.slots = a->head_dim <= 128 ? 2 * kCus : kCus;   // the kernel's launch bounds
-            p.min_chunk = a->in_dtype == TV_F32 ? kMinChunk32 : kMinChunk16;
+            p.slots = chip_slots(a->head_dim);
+            p.min_chunk = min_chunk_tiles(a->in_dtype);
             // (maximum, sum) pairs first: 8-byte aligned whatever the head size.
             p.ws_ml = static_cast<float2*>(workspace);
             p.ws_o = reinterpret_cast<float*>(p.ws_ml + units * splits * kBlockRows);
