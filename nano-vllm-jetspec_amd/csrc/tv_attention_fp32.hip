@@ -81,13 +81,14 @@ struct Fp32Params {
     float scale;          // softmax scale * log2(e) / 2: scores are kept in kUnit
     int32_t splits;       // chunks a row block's keys may be cut into
     int32_t slots;        // workgroups the chip runs at a time
+    int32_t places;       // workgroups of a cut launch, each with room for its partial rows
     int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
     int32_t kv_heads;
     int32_t vec;          // K/V rows take vector loads
     int32_t q_vec;        // Q rows do
     int64_t unit0;        // first (row block, KV head) of this launch
-    float* ws_o;          // partial rows [row group, KV head, split, 32, head_dim] (splits > 1)
-    float2* ws_ml;        // their (maximum, sum) [row group, KV head, split, 32]
+    float* ws_o;          // partial rows [chunk, KV head, 32, head_dim] (splits > 1)
+    float2* ws_ml;        // their (maximum, sum) [chunk, KV head, 32]
     int32_t* status;
 };
 
@@ -113,7 +114,7 @@ constexpr int kWaves = 4;           // waves of a workgroup: they take its tiles
 constexpr int kThreadsFp32 = kWave * kWaves;
 constexpr int kMaxSplits = 16;
 constexpr int kCus = 256;           // compute units of an MI355X
-constexpr int64_t kCutRows = 4096;  // partial row blocks a workspace holds at most
+constexpr int64_t kCutRows = 4096;  // row blocks times chunks a batch is cut into at most
 constexpr int kCutRequests = kWave; // requests of a batch that is cut at most (one lane each)
 // Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
 // rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
@@ -154,10 +155,10 @@ __device__ int request_of_group(const int32_t* cu, int groups, int num_requests,
 struct RowBlock {
     int r, row0, rows, nodes, prefix;   // rows: score rows of the block (<= 32)
     int64_t tree0;                      // the request's first packed row
-    int64_t number;                     // the block's number (group_start), which places its partial rows
     int tiles;                          // 32-key tiles any row of the block can see
     int seq;                            // ... keys
     int chunk, part;                    // tiles of a chunk, this workgroup's chunk
+    int first;                          // index of the block's first chunk, which places its partial rows
 };
 
 // Fills the block `index` of request r, whose live metadata are given; false for an index past
@@ -169,7 +170,7 @@ __device__ __forceinline__ bool block_of_request(const Fp32Params& p, int r, int
     b.prefix = prefix;
     b.nodes = nodes;
     b.tree0 = cu;
-    b.number = static_cast<int64_t>(cu) * p.groups / kBlockRows + r + index;
+    b.first = 0;
     const int64_t rows = static_cast<int64_t>(nodes) * p.groups;
     if (b.row0 >= rows) return false;
     const int last = static_cast<int>((min(static_cast<int64_t>(b.row0) + kBlockRows, rows) - 1) / p.groups);
@@ -301,6 +302,7 @@ __device__ __forceinline__ bool cut_block(const Fp32Params& p, const Cut& cut, i
     if (live) {
         b.chunk = chunk_tiles(__builtin_amdgcn_readlane(cut.tiles, l), np);
         b.part = index - block * np;
+        b.first = u - b.part;
         live = b.part * b.chunk < b.tiles;   // an early block sees fewer keys than its request holds
     }
     return true;
@@ -784,7 +786,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
     }
     __syncthreads();
     const bool split = b.tiles > b.chunk;   // this block has further chunks
-    const int64_t part = ((b.number * p.kv_heads + kvh) * p.splits + b.part) * kBlockRows;
+    const int64_t part = (static_cast<int64_t>(b.first + b.part) * p.kv_heads + kvh) * kBlockRows;
     if (split && tid < kBlockRows) {
         float sum = 0.f;
 #pragma unroll
@@ -839,16 +841,17 @@ tree_attention_fp32_kernel(const Fp32Params p) {
         }
         return;
     }
+    // The cut has at most p.places workgroups unless the live metadata hold more row blocks than
+    // the launch's shapes allow.
     const Cut cut = plan_cut(p);
-    for (int i = blockIdx.x;; i += gridDim.x) {
-        const int u = i / p.kv_heads;
-        bool live;
-        if (!cut_block(p, cut, u, b, live)) return;
-        if (live) {
-            attend_block<T, DIM, EXACT>(p, b, i - u * p.kv_heads);
-            __syncthreads();   // the next block reuses the LDS
-        }
+    const int u = blockIdx.x / p.kv_heads;
+    if (blockIdx.x == 0) {
+        const int chunks = wave_total(cut.blocks * chunks_of(cut.tiles, cut.target));
+        if (static_cast<int64_t>(chunks) * p.kv_heads > p.places) set_status(p.status, TV_STATUS_BAD_REQUEST);
     }
+    bool live;
+    if (!cut_block(p, cut, u, b, live) || !live) return;
+    attend_block<T, DIM, EXACT>(p, b, blockIdx.x - u * p.kv_heads);
 }
 
 // Combines the chunks of the row blocks that were cut: one wave per score row, its partial
@@ -863,23 +866,28 @@ merge_fp32_kernel(const Fp32Params p) {
                         static_cast<int64_t>(cut.cu) * p.groups / kBlockRows + lane <= number;
     const int r = 63 - __builtin_clzll(__ballot(before) | 1ull);
     const int cu = __builtin_amdgcn_readlane(cut.cu, r), tiles = __builtin_amdgcn_readlane(cut.tiles, r);
+    const int np = chunks_of(tiles, cut.target), mine = cut.blocks * chunks_of(cut.tiles, cut.target);
+    const int before_r = __builtin_amdgcn_readlane(prefix_sum(mine) - mine, r);   // chunks of the earlier requests
+    const int index = number - static_cast<int>(static_cast<int64_t>(cu) * p.groups / kBlockRows + r);
     RowBlock b;
-    if (!block_of_request(p, r, number - static_cast<int>(static_cast<int64_t>(cu) * p.groups / kBlockRows + r), cu,
+    if (!block_of_request(p, r, index, cu,
                           __builtin_amdgcn_readlane(cut.nodes, r), __builtin_amdgcn_readlane(cut.prefix, r), b, false) ||
         tiles == 0) {
         return;
     }
-    const int chunk = chunk_tiles(tiles, chunks_of(tiles, cut.target));
+    const int chunk = chunk_tiles(tiles, np);
     if (b.tiles <= chunk) return;   // one chunk: the attention kernel wrote the rows
     const int parts = (b.tiles + chunk - 1) / chunk;
-    const int64_t first = (b.number * p.kv_heads + kvh) * p.splits * kBlockRows;
+    const int64_t step = static_cast<int64_t>(p.kv_heads) * kBlockRows;   // rows from a chunk to the next
+    const int64_t first = (static_cast<int64_t>(before_r) + static_cast<int64_t>(index) * np) * step + kvh * kBlockRows;
+    if (first + (parts - 1) * step >= static_cast<int64_t>(p.places) * kBlockRows) return;   // reported: no such workgroup
     const int rr = blockIdx.y * kWaves + threadIdx.x / kWave;
     if (rr >= b.rows) return;
     const int node = (b.row0 + rr) / p.groups, head = kvh * p.groups + (b.row0 + rr) % p.groups;
     const int64_t at = b.tree0 + node;
     if (p.q2r[at] != r || p.local[at] != node) return;
     // Lane s holds partial s's maximum and sum.
-    const float2 ml = lane < parts ? p.ws_ml[first + lane * kBlockRows + rr] : make_float2(-INFINITY, 0.f);
+    const float2 ml = lane < parts ? p.ws_ml[first + lane * step + rr] : make_float2(-INFINITY, 0.f);
     float top = ml.x;
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
@@ -897,7 +905,7 @@ merge_fp32_kernel(const Fp32Params p) {
             float x[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                x[s] = s0 + s < parts ? p.ws_o[(first + (s0 + s) * kBlockRows + rr) * p.head_dim + dl] : 0.f;
+                x[s] = s0 + s < parts ? p.ws_o[(first + (s0 + s) * step + rr) * p.head_dim + dl] : 0.f;
             }
 #pragma unroll
             for (int s = 0; s < 8; ++s) o = fmaf(x[s], __shfl(w, s0 + s), o);   // w is 0 past the parts
@@ -920,8 +928,13 @@ int64_t blocks_of(int64_t nodes, int64_t groups) { return (nodes * groups + kBlo
 // Workgroups the chip runs at a time (the kernel's launch bounds) and the shortest chunk.
 int chip_slots(int32_t head_dim) { return head_dim <= 128 ? 2 * kCus : kCus; }
 int min_chunk_tiles(int32_t in_dtype) { return in_dtype == TV_F32 ? kMinChunk32 : kMinChunk16; }
-int64_t partial_bytes(int64_t units, int splits, int32_t head_dim) {
-    return units * splits * kBlockRows * (static_cast<int64_t>(head_dim) * 4 + static_cast<int64_t>(sizeof(float2)));
+// Workgroups of a cut launch: the chip's slots, as many times as the row blocks fill them.
+int64_t cut_places(int64_t units, int32_t head_dim) {
+    const int64_t slots = chip_slots(head_dim);
+    return slots * ((units + slots - 1) / slots);
+}
+int64_t partial_bytes(int64_t places, int32_t head_dim) {
+    return places * kBlockRows * (static_cast<int64_t>(head_dim) * 4 + static_cast<int64_t>(sizeof(float2)));
 }
 
 // Rows the vector loads take: unit element stride, 16-byte aligned rows, and a head size
@@ -940,8 +953,7 @@ void launch_for_dims(const Fp32Params& p, const dim3& grid, hipStream_t s) {
 // The head sizes models use are compiled in; the others share an instance per power of two.
 template <typename T>
 void launch_for_type(const Fp32Params& p, uint32_t units, hipStream_t s) {
-    // Cut: the blocks' first chunks and the chip's slots; workgroups loop where that is too few.
-    const dim3 grid(p.splits == 1 ? units : units + p.slots);
+    const dim3 grid(p.splits == 1 ? units : static_cast<uint32_t>(p.places));
     const int d = p.head_dim;
     if (p.vec && d == 64) {
         launch_for_dims<T, 64, true>(p, grid, s);
@@ -988,7 +1000,7 @@ extern "C" int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries,
     const int64_t groups = num_q_heads / num_kv_heads;
     const int splits = split_count(total_queries, num_requests, groups, num_kv_heads);
     if (splits == 1) return 0;
-    return partial_bytes(row_groups(total_queries, num_requests, groups) * num_kv_heads, splits, head_dim);
+    return partial_bytes(cut_places(row_groups(total_queries, num_requests, groups) * num_kv_heads, head_dim), head_dim);
 }
 
 extern "C" int tv_tree_attention_fp32_chunk_keys(const int32_t* prefix_lens_host, const int32_t* node_counts_host,
@@ -1121,16 +1133,18 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
         const int splits = split_count(a->total_queries, a->num_requests, p.groups, a->num_kv_heads);
         if (splits > 1) {
             if (!aligned(workspace, 16)) return fail(TV_ERR_INVALID, "tree_attention_fp32: unaligned workspace");
-            if (workspace_bytes < partial_bytes(units, splits, a->head_dim)) {
+            const int64_t places = cut_places(units, a->head_dim), bytes = partial_bytes(places, a->head_dim);
+            if (workspace_bytes < bytes) {
                 return fail(TV_ERR_CAPACITY, "tree_attention_fp32: workspace of %lld bytes, %lld needed",
-                            (long long)workspace_bytes, (long long)partial_bytes(units, splits, a->head_dim));
+                            (long long)workspace_bytes, (long long)bytes);
             }
+            p.places = static_cast<int32_t>(places);
             p.splits = splits;
             p.slots = chip_slots(a->head_dim);
             p.min_chunk = min_chunk_tiles(a->in_dtype);
             // (maximum, sum) pairs first: 8-byte aligned whatever the head size.
             p.ws_ml = static_cast<float2*>(workspace);
-            p.ws_o = reinterpret_cast<float*>(p.ws_ml + units * splits * kBlockRows);
+            p.ws_o = reinterpret_cast<float*>(p.ws_ml + places * kBlockRows);
         }
     }
     hipStream_t s = as_stream(stream);

@@ -173,12 +173,18 @@ def _fp32_template(metadata, k_pool, v_pool, queries_per_kv: int, device):
 
 def _enqueue_fp32(a, device, stream: int, what: str) -> None:
     """Launch a complete FP32-kernel block.  A batch of few score rows cuts its keys over several
-    workgroups through a workspace that lives for this call only, as any temporary of the
-    stream (or of the graph being captured): no two launches share one."""
+    workgroups through a workspace (8.5 MB at head size 128 while the row blocks fit the chip at
+    once) that lives for this call only, as any temporary of the stream (or of the graph being
+    captured): no two launches share one.  Without memory for it the keys stay whole."""
     lib = _lib.library()
     size = int(lib.tv_tree_attention_fp32_workspace_bytes(a.total_queries, a.num_requests, a.num_q_heads,
                                                           a.num_kv_heads, a.head_dim))
-    workspace = torch.empty(size, dtype=torch.uint8, device=device) if size else None
+    workspace = None
+    if size:
+        try:
+            workspace = torch.empty(size, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            size = 0
     _lib.check(lib.tv_tree_attention_fp32_split(ctypes.byref(a), workspace.data_ptr() if size else None, size, stream),
                what)
 

@@ -78,3 +78,14 @@ def test_invalid_lengths_are_refused():
     for prefixes, nodes in (([-1], [4]), ([4], [-1]), ([2 ** 31 - 1], [4])):
         with pytest.raises(Exception, match="invalid lengths"):
             cut(prefixes, nodes, 4, 1, 128, _lib.TV_F32)
+
+
+def test_the_workspace_holds_one_partial_block_per_workgroup():
+    """Sized by the workgroups the chip runs at a time, whatever the head count or chunks."""
+    size = _lib.library().tv_tree_attention_fp32_workspace_bytes
+    for queries, requests, q_heads, kv_heads, dim in ((64, 1, 32, 8, 128), (200, 8, 24, 8, 96), (1, 1, 1, 1, 512),
+                                                      (400, 64, 32, 8, 192), (3000, 2, 4, 1, 80)):
+        blocks = (queries * (q_heads // kv_heads) // BLOCK + requests + 1) * kv_heads
+        slots = 512 if dim <= 128 else 256
+        assert size(queries, requests, q_heads, kv_heads, dim) == -(-blocks // slots) * slots * BLOCK * (4 * dim + 8)
+    assert size(64, 65, 32, 8, 128) == 0 and size(40000, 2, 32, 8, 128) == 0

@@ -45,3 +45,21 @@ def test_a_request_without_nodes_among_live_metadata():
     error, _ = errors(out, oracle_rows(q, k, v, meta, 96 ** -0.5, [0, 2]))
     assert error <= BOUND
     assert read_and_clear_status(DEV) == 0
+
+
+def test_without_memory_for_the_workspace_the_keys_stay_whole(monkeypatch):
+    q, k, v, meta, *_ = make_case((900, 1500), (9, 30), head_dim=96, dtype=torch.float32, seed=6)
+    real = torch.empty
+
+    def full(*args, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return real(*args, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    out = packed_tree_attention(q, k, v, meta, 96 ** -0.5, 4)
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    error, _ = errors(out, oracle_rows(q, k, v, meta, 96 ** -0.5, [0, 1]))
+    assert error <= BOUND
+    assert read_and_clear_status(DEV) == 0
