@@ -566,6 +566,17 @@ int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries, int32_t nu
 int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* args, void* workspace,
                                  int64_t workspace_bytes, void* stream);
 /*
+ * The same for a caller that knows the batch's longest request on the host: max_keys is its prefix
+ * and nodes (0: unknown, as tv_tree_attention_fp32_split).  Short batches then take one launch of
+ * the form that is faster for them and no workspace.  The number chooses the launches and nothing
+ * else: the kernels compute any live lengths, and with the true one the same bits as without.
+ */
+int64_t tv_tree_attention_fp32_keys_workspace_bytes(int32_t total_queries, int32_t num_requests,
+                                                    int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                                    int32_t in_dtype, int32_t max_keys);
+int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* args, int32_t max_keys, void* workspace,
+                                int64_t workspace_bytes, void* stream);
+/*
  * How a launch with a workspace cuts a batch of these lengths (host arrays): the longest chunk of
  * a row block's keys (0: batches of this shape are never cut) and the workgroups that have work.
  * The kernel takes the same decision from the live lengths.

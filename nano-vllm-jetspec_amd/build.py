@@ -32,7 +32,7 @@ ATTENTION_GROUP_SOURCES = (tuple(f"tv_attention_g{g}.hip" for g in GROUPS) +
                            tuple(f"tv_attention_d64_g{g}.hip" for g in GROUPS_D64) +
                            tuple(f"tv_attention_d256_g{g}.hip" for g in GROUPS_D256))
 SOURCES = ("tv_common.cpp", "tv_plan.cpp", "tv_kvcache.hip", "tv_attention.hip", *ATTENTION_GROUP_SOURCES,
-           "tv_attention_fp32.hip",
+           "tv_attention_fp32.hip", "tv_attention_rows.hip",
            "tv_rope.hip", "tv_accept.hip", "tv_metadata.hip", "tv_plan_device.hip")
 
 # Packed-FP32 VALU instructions are kept out of the device code (they are not

@@ -44,69 +44,10 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "tv_internal.h"
+#include "tv_attention_fp32.h"
 
 namespace tv {
 namespace {
-
-struct Fp32Params {
-    const void* q;
-    int64_t q_s0, q_s1;
-    const void* k;
-    const void* v;
-    int64_t k_s0, k_s1, k_s2, k_s3;
-    int64_t v_s0, v_s1, v_s2, v_s3;
-    int64_t num_blocks;
-    void* out;
-    int64_t o_s0, o_s1;
-    int32_t out_dtype;
-    const int32_t* cu;
-    const int32_t* q2r;
-    const int32_t* local;
-    const int32_t* plen;
-    const int32_t* cnt;
-    const int32_t* tables;
-    int64_t t_s0;
-    const int64_t* tree_slots;
-    const float* bias;
-    const int64_t* bias_off;
-    const void* pslots;
-    int64_t ps_s0;
-    int32_t ps_i64;
-    int32_t num_requests;
-    int32_t total_queries;
-    int32_t groups;       // query heads per KV head
-    int32_t head_dim;
-    int32_t block_size;
-    float scale;          // softmax scale * log2(e) / 2: scores are kept in kUnit
-    int32_t splits;       // chunks a row block's keys may be cut into
-    int32_t slots;        // workgroups the chip runs at a time
-    int32_t places;       // workgroups of a cut launch, each with room for its partial rows
-    int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
-    int32_t kv_heads;
-    int32_t vec;          // K/V rows take vector loads
-    int32_t q_vec;        // Q rows do
-    int64_t unit0;        // first (row block, KV head) of this launch
-    float* ws_o;          // partial rows [chunk, KV head, 32, head_dim] (splits > 1)
-    float2* ws_ml;        // their (maximum, sum) [chunk, KV head, 32]
-    int32_t* status;
-};
-
-constexpr int kWave = 64;
-
-__device__ __forceinline__ float to_float(float x) { return x; }
-__device__ __forceinline__ float to_float(__bf16 x) { return static_cast<float>(x); }
-__device__ __forceinline__ float to_float(_Float16 x) { return static_cast<float>(x); }
-
-__device__ __forceinline__ void store_value(const Fp32Params& p, int64_t index, float x) {
-    if (p.out_dtype == TV_F32) {
-        static_cast<float*>(p.out)[index] = x;
-    } else if (p.out_dtype == TV_BF16) {
-        static_cast<__bf16*>(p.out)[index] = static_cast<__bf16>(x);
-    } else {
-        static_cast<_Float16*>(p.out)[index] = static_cast<_Float16>(x);
-    }
-}
 
 constexpr int kBlockRows = 32;      // score rows of a workgroup
 constexpr int kTile = 32;           // keys of a tile
@@ -119,6 +60,8 @@ constexpr int kCutRequests = kWave; // requests of a batch that is cut at most (
 // Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
 // rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
 constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
+constexpr int32_t kMaxRowKeys = 256;    // the most keys of a request the row form takes
+constexpr int64_t kRowRequests = 1024;  // ... and requests (every workgroup reads the lengths of a captured launch)
 // Scores and maxima are kept in units of two octaves (natural units * log2(e) / 2): the factor is
 // below 1, so that the most negative bias a mask can hold stays a finite score (in log2 units
 // torch.finfo(float32).min would become -inf and a row that sees nothing else a NaN).
@@ -828,6 +771,7 @@ __device__ __forceinline__ void attend_block(const Fp32Params& p, const RowBlock
 template <typename T, int DIM, bool EXACT>
 __global__ void __launch_bounds__(kThreadsFp32, DIM <= 128 ? 2 : 1)
 tree_attention_fp32_kernel(const Fp32Params p) {
+    if (p.rows_keys > 0 && longest_request(p) <= p.rows_keys) return;   // the row form's batch
     // Index -> (block, chunk) and KV head, head fastest: with 8 KV heads the blocks and chunks of one
     // head share an XCD (workgroup i runs on XCD i % 8), and so its K/V in that L2.
     RowBlock b;
@@ -928,6 +872,34 @@ int64_t blocks_of(int64_t nodes, int64_t groups) { return (nodes * groups + kBlo
 // Workgroups the chip runs at a time (the kernel's launch bounds) and the shortest chunk.
 int chip_slots(int32_t head_dim) { return head_dim <= 128 ? 2 * kCus : kCus; }
 int min_chunk_tiles(int32_t in_dtype) { return in_dtype == TV_F32 ? kMinChunk32 : kMinChunk16; }
+// Head sizes with an instance of their own (vector rows only).
+bool own_instance(int32_t d) {
+    return d == 64 || d == 80 || d == 96 || d == 112 || d == 128 || d == 192 || d == 256;
+}
+// Keys of the longest request up to which a batch takes the row form (0: never), from the launch's
+// shapes.  The row form's time grows with 64-key tiles (f32, head size 128, one query head a KV
+// head: 5 + 5.5 us a tile; four: 7 + 7.5; eight: 11 + 19, always behind), the matrix form's hardly
+// within 128 keys (14 us with one score row a request, 20 with 32).  us, row / matrix form, one
+// request of 8 KV heads: f32 x 128, 64 keys, 24 rows 10.3 / 20.2; 192 keys, 64 rows 22 / 29; 248
+// keys, 8 rows 27 / 24; four heads a KV head, 120 keys, 40 nodes 20.7 / 23.3; 192 keys 29.5 / 29.5;
+// f32 x 64, 64 keys, 24 rows 8 / 16.  In 16 bits the instances of their own are ahead from a few
+// dozen keys on (x 96, three heads: always; x 80, one head, 64 keys, 24 rows 13 / 18), the shared
+// ones, with their padding and element loads, behind for longer (x 72, 192 keys, 64 rows 28 / 35).
+// Beyond one round of its workgroups (two a CU) the row form loses its lead unless the matrix
+// form's are about as many (48 requests of 8 nodes, four heads: 36 / 54; of 24 nodes 83 / 85).
+int32_t row_form_keys(int64_t total_queries, int64_t num_requests, int64_t groups, int64_t kv_heads, int32_t in_dtype,
+                      int32_t head_dim, bool vec) {
+    if (groups > 4 || num_requests > kRowRequests) return 0;
+    const int64_t row_groups_4 = (total_queries / 4 + num_requests + 1) * kv_heads;
+    if (row_groups_4 > 2 * kCus && 2 * row_groups_4 > 3 * row_groups(total_queries, num_requests, groups) * kv_heads) return 0;
+    const bool own = vec && own_instance(head_dim), f32 = in_dtype == TV_F32, few_heads = groups <= 2;
+    const bool full = total_queries * groups >= 20 * num_requests;   // score rows of the average request
+    if (!f32 && own) return few_heads ? (full ? (head_dim <= 128 ? 64 : 0) : 32) : 0;
+    if (head_dim > 128) return few_heads ? 64 : (full ? 0 : 32);
+    const bool longer = f32 && (head_dim > 64 || !own);
+    if (few_heads) return longer ? (full ? 256 : 128) : (full ? 192 : 64);
+    return full ? (longer ? (own ? 128 : 192) : 64) : 32;
+}
 // Workgroups of a cut launch: the chip's slots, as many times as the row blocks fill them.
 int64_t cut_places(int64_t units, int32_t head_dim) {
     const int64_t slots = chip_slots(head_dim);
@@ -1003,6 +975,13 @@ extern "C" int64_t tv_tree_attention_fp32_workspace_bytes(int32_t total_queries,
     return partial_bytes(cut_places(row_groups(total_queries, num_requests, groups) * num_kv_heads, head_dim), head_dim);
 }
 
+extern "C" int64_t tv_tree_attention_fp32_keys_workspace_bytes(int32_t total_queries, int32_t num_requests,
+                                                               int32_t num_q_heads, int32_t num_kv_heads,
+                                                               int32_t head_dim, int32_t in_dtype, int32_t max_keys) {
+    if (max_keys > 0 && max_keys <= min_chunk_tiles(in_dtype) * kTile) return 0;   // never cut
+    return tv_tree_attention_fp32_workspace_bytes(total_queries, num_requests, num_q_heads, num_kv_heads, head_dim);
+}
+
 extern "C" int tv_tree_attention_fp32_chunk_keys(const int32_t* prefix_lens_host, const int32_t* node_counts_host,
                                                  int32_t num_requests, int32_t num_q_heads, int32_t num_kv_heads,
                                                  int32_t head_dim, int32_t in_dtype, int32_t* chunk_keys,
@@ -1052,11 +1031,16 @@ extern "C" int tv_tree_attention_fp32_chunk_keys(const int32_t* prefix_lens_host
 }
 
 extern "C" int tv_tree_attention_fp32(const tv_tree_attention_fp32_args* a, void* stream) {
-    return tv_tree_attention_fp32_split(a, nullptr, 0, stream);
+    return tv_tree_attention_fp32_keys(a, 0, nullptr, 0, stream);
 }
 
 extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a, void* workspace,
                                             int64_t workspace_bytes, void* stream) {
+    return tv_tree_attention_fp32_keys(a, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* a, int32_t max_keys, void* workspace,
+                                           int64_t workspace_bytes, void* stream) {
     clear_error();
     if (!a) return fail(TV_ERR_INVALID, "tree_attention_fp32: null args");
     if (a->num_requests < 1 || a->total_queries < 0) return fail(TV_ERR_INVALID, "tree_attention_fp32: invalid counts");
@@ -1080,6 +1064,7 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
     if (a->prefix_slots && a->prefix_slots_stride < 0) {
         return fail(TV_ERR_INVALID, "tree_attention_fp32: negative prefix slot stride");
     }
+    if (max_keys < 0) return fail(TV_ERR_INVALID, "tree_attention_fp32: negative key count");
     if (a->total_queries == 0) return TV_OK;
     if (!a->q || !a->k_pool || !a->v_pool || !a->out || !a->cu_seqlens_q || !a->query_to_request ||
         !a->query_local_row || !a->prefix_lens || !a->node_counts || !a->tree_slots || !a->qq_bias ||
@@ -1129,7 +1114,7 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
     p.splits = 1;
     p.ws_o = nullptr;
     p.ws_ml = nullptr;
-    if (workspace) {
+    if (workspace && (max_keys == 0 || max_keys > min_chunk_tiles(a->in_dtype) * kTile)) {
         const int splits = split_count(a->total_queries, a->num_requests, p.groups, a->num_kv_heads);
         if (splits > 1) {
             if (!aligned(workspace, 16)) return fail(TV_ERR_INVALID, "tree_attention_fp32: unaligned workspace");
@@ -1147,12 +1132,25 @@ extern "C" int tv_tree_attention_fp32_split(const tv_tree_attention_fp32_args* a
             p.ws_o = reinterpret_cast<float*>(p.ws_ml + places * kBlockRows);
         }
     }
-    hipStream_t s = as_stream(stream);
     const int64_t elem = a->in_dtype == TV_F32 ? 4 : 2;
     p.vec = vector_rows(a->k_pool, a->k_stride, elem, a->head_dim) &&
             vector_rows(a->v_pool, a->v_stride, elem, a->head_dim);
     const int64_t per = 16 / elem;
     p.q_vec = aligned(a->q, 16) && a->q_stride_row % per == 0 && a->q_stride_head % per == 0 && a->head_dim % per == 0;
+    // A batch whose lengths the host knows takes its form here; otherwise both are launched and
+    // the one that is not the batch's exits.
+    hipStream_t s = as_stream(stream);
+    const int32_t rows_keys = row_form_keys(a->total_queries, a->num_requests, p.groups, a->num_kv_heads, a->in_dtype,
+                                            a->head_dim, p.vec);
+    static_assert(kMaxRowKeys <= kTile * kMinChunk32 && kMaxRowKeys <= kTile * kMinChunk16, "such a batch is never cut");
+    p.rows_keys = 0;
+    if (rows_keys > 0 && max_keys <= rows_keys) {
+        Fp32Params rows = p;
+        rows.scale = a->scale;
+        if (max_keys == 0) rows.rows_keys = p.rows_keys = rows_keys;
+        launch_rows(rows, a->in_dtype, s);
+        if (max_keys > 0) return check_launch("tree_attention_fp32");
+    }
     // A grid holds 2^32 threads: a huge batch takes several launches.
     constexpr int64_t kLaunchUnits = int64_t{1} << 23;
     for (p.unit0 = 0; p.unit0 < units; p.unit0 += kLaunchUnits) {

@@ -67,6 +67,8 @@ EXPORTED_SYMBOLS = (
     "tv_tree_attention_fp32_split",
     "tv_tree_attention_fp32_workspace_bytes",
     "tv_tree_attention_fp32_chunk_keys",
+    "tv_tree_attention_fp32_keys",
+    "tv_tree_attention_fp32_keys_workspace_bytes",
 )
 
 
@@ -240,6 +242,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tv_tree_attention_fp32_split.argtypes = [POINTER(TreeAttentionFp32Args), c_void_p, c_int64, c_void_p]
     lib.tv_tree_attention_fp32_workspace_bytes.restype = c_int64
     lib.tv_tree_attention_fp32_workspace_bytes.argtypes = [c_int32] * 5
+    lib.tv_tree_attention_fp32_keys.restype = c_int32
+    lib.tv_tree_attention_fp32_keys.argtypes = [POINTER(TreeAttentionFp32Args), c_int32, c_void_p, c_int64, c_void_p]
+    lib.tv_tree_attention_fp32_keys_workspace_bytes.restype = c_int64
+    lib.tv_tree_attention_fp32_keys_workspace_bytes.argtypes = [c_int32] * 7
     lib.tv_tree_attention_fp32_chunk_keys.restype = c_int32
     lib.tv_tree_attention_fp32_chunk_keys.argtypes = [POINTER(c_int32), POINTER(c_int32), *[c_int32] * 5,
                                                       POINTER(c_int32), POINTER(c_int32)]

@@ -171,25 +171,28 @@ def _fp32_template(metadata, k_pool, v_pool, queries_per_kv: int, device):
     return a
 
 
-def _enqueue_fp32(a, device, stream: int, what: str) -> None:
+def _enqueue_fp32(a, device, stream: int, max_keys: int, what: str) -> None:
     """Launch a complete FP32-kernel block.  A batch of few score rows cuts its keys over several
     workgroups through a workspace (8.5 MB at head size 128 while the row blocks fit the chip at
     once) that lives for this call only, as any temporary of the stream (or of the graph being
-    captured): no two launches share one.  Without memory for it the keys stay whole."""
+    captured): no two launches share one.  Without memory for it the keys stay whole.  `max_keys`
+    is the longest request's prefix and nodes; a launch being captured follows the live ones."""
     lib = _lib.library()
-    size = int(lib.tv_tree_attention_fp32_workspace_bytes(a.total_queries, a.num_requests, a.num_q_heads,
-                                                          a.num_kv_heads, a.head_dim))
+    if torch.cuda.is_current_stream_capturing():
+        max_keys = 0
+    size = int(lib.tv_tree_attention_fp32_keys_workspace_bytes(
+        a.total_queries, a.num_requests, a.num_q_heads, a.num_kv_heads, a.head_dim, a.in_dtype, max_keys))
     workspace = None
     if size:
         try:
             workspace = torch.empty(size, dtype=torch.uint8, device=device)
         except torch.OutOfMemoryError:
             size = 0
-    _lib.check(lib.tv_tree_attention_fp32_split(ctypes.byref(a), workspace.data_ptr() if size else None, size, stream),
-               what)
+    _lib.check(lib.tv_tree_attention_fp32_keys(ctypes.byref(a), max_keys, workspace.data_ptr() if size else None, size,
+                                               stream), what)
 
 
-def _launch_fp32(a, q, out, scale, stream: int) -> torch.Tensor:
+def _launch_fp32(a, q, out, scale, stream: int, max_keys: int = 0) -> torch.Tensor:
     """Complete a copy of an FP32-kernel argument block with Q, O and scale, and launch."""
     a = _lib.TreeAttentionFp32Args.from_buffer_copy(a)
     if q.stride(-1) != 1 or out.stride(-1) != 1:
@@ -200,7 +203,7 @@ def _launch_fp32(a, q, out, scale, stream: int) -> torch.Tensor:
     a.out_stride_row, a.out_stride_head = out.stride(0), out.stride(1)
     a.out_dtype = _device.dtype_code(out.dtype)
     a.scale = float(scale)
-    _enqueue_fp32(a, q.device, stream, "tree_attention_fp32")
+    _enqueue_fp32(a, q.device, stream, max_keys, "tree_attention_fp32")
     return out
 
 
@@ -409,14 +412,15 @@ def _launch(q, k_pool, v_pool, metadata, scale, out, *, chunk_keys: int = 0, exa
     entry = per_meta.get(key)
     if entry is None:
         if not _mfma_geometry(q, k_pool, v_pool, metadata):
-            entry = per_meta[key] = (_FP32_ROUTE, _fp32_template(metadata, k_pool, v_pool, queries_per_kv, q.device))
+            keys = max(p + n for p, n in zip(metadata.prefix_lengths, metadata.node_counts_host))
+            entry = per_meta[key] = (_FP32_ROUTE, _fp32_template(metadata, k_pool, v_pool, queries_per_kv, q.device), keys)
         elif torch.cuda.is_current_stream_capturing():
             entry = None
         else:
             entry = per_meta[key] = _eager_template(per_meta, metadata, k_pool, v_pool, num_kv_heads,
                                                     queries_per_kv, chunk_keys, stream)
     if entry is not None and entry[0] is _FP32_ROUTE:
-        return _launch_fp32(entry[1], q, out, scale, stream)
+        return _launch_fp32(entry[1], q, out, scale, stream, entry[2])
     if q.stride(0) % 8 or q.stride(1) % 8 or q.data_ptr() % 16:
         q = q.contiguous()
     if torch.cuda.is_current_stream_capturing():
@@ -588,7 +592,8 @@ def _legacy_fp32(q, k_pool, v_pool, req, scale, block_size: int, out, device) ->
     a.block_size = block_size
     a.scale = float(scale)
     a.status = _device.status_word(device).data_ptr()
-    _enqueue_fp32(a, device, _device.stream_handle(device), "tree_attention_fp32 (slot addressed)")
+    _enqueue_fp32(a, device, _device.stream_handle(device), req.prefix + req.total_q,
+                  "tree_attention_fp32 (slot addressed)")
 
 
 def _legacy_mfma(q, k_pool, v_pool, req, scale, num_queries_per_kv: int, block_size: int, out, device) -> None:
