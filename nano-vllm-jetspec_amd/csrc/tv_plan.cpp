@@ -9,15 +9,15 @@
 // so a KV tile staged in LDS is reused by every (node, query head) row of its group.
 // Long prefixes are cut into chunks (split-K) only as far as needed to give every
 // compute unit work; items are ordered longest first so the hardware dispatcher's
-// greedy assignment balances ragged contexts (an LPT schedule).  Up to kFillRounds
-// rounds of items, the chunk target is the smallest whose items fit a chosen number of
-// whole rounds (see kRoundCost), so no round is part-empty.
+// greedy assignment balances ragged contexts (an LPT schedule).  Two to kFillRounds rounds
+// of items are made whole rounds, as many or fewer (plan_target).
 #include <stdint.h>
 
 #include <algorithm>
 #include <vector>
 
 #include "tv_internal.h"
+#include "tv_plan_rule.h"
 
 namespace tv {
 namespace {
@@ -25,43 +25,10 @@ namespace {
 constexpr int kItemInts = 8;
 constexpr int kRowsPerItem = 256;   // score rows of one workgroup
 constexpr int kHeadDim = 128;
-constexpr int kMinChunkKeys = 64;   // shortest prefix chunk worth a partial result
 constexpr int kMaxChunkPages = 512; // page numbers a workgroup caches in LDS
 constexpr int kMaxSlotChunk = 2048; // prefix slots a workgroup caches in LDS (slot addressing)
 constexpr int kMaxTreeNodes = 2048; // tree slots a workgroup caches in LDS (page-table prefixes)
 constexpr int kMaxTreeNodesSlots = 1024;   // ... beside a slot-addressed prefix chunk
-constexpr int64_t kFillRounds = 4;  // item rounds the chunk target is chosen for
-
-// Choice of the chunk target, in cost units (about 142 a microsecond).  A batch that fits one
-// round gets as many items as balance its streaming against its partial results: n items of
-// an even share stream total / n, and each writes and the merge reads 133 KB, about
-// kPartialCost, so n = sqrt(total / kPartialCost), at most one per compute unit.  A batch that
-// does not fit one round when every item has the even share of a compute unit takes the number
-// of whole rounds whose estimated span is the smallest: a round costs its longest item and
-// kRoundCost (the item's lookups, first loads and stores, 8 us), a slot kSlotCost (what of its
-// merge the launch does not hide).  8 requests of 1354-4060 keys and 18-54 nodes, 8 KV heads:
-// 496 items in two rounds 64.5 us, 244 in one 49.1; a one-head shard of 32 requests of
-// 1.1k-8.1k keys: 499 items 75.8 us, 227 items 53.9; 8 requests of 545-1603 keys and 32 nodes:
-// 236 items 29.9 us, 160 items 27.9.
-// kPartialCost of 3, 5 and 8, us: 8 requests of 1390-3225 keys on 2 KV heads 30.5, 29.0, 30.5
-// (204, 156, 138 items); 4 requests of 500-2000 keys on one 23.7, 21.6, 23.0; 16 of 2-8k keys on
-// one 30.9, 30.9, 31.8; 8 of 256-2048 keys on 8 29.2, 28.0, 28.5.
-constexpr int64_t kPartialCost = 5;
-constexpr int64_t kRoundCost = 1000;
-constexpr int64_t kSlotCost = 2;
-constexpr int64_t kTauStep = 128;   // 32 keys of a one-head item
-
-int64_t one_round_items(int64_t total_cost, int64_t units, int64_t compute_units) {
-    const int64_t x = total_cost / kPartialCost;
-    int64_t n = compute_units;
-    if (x < compute_units * compute_units) {
-        n = 0;
-        for (int64_t bit = int64_t{1} << 20; bit > 0; bit >>= 1) {   // integer square root
-            if ((n + bit) * (n + bit) <= x) n += bit;
-        }
-    }
-    return std::min(compute_units, std::max(n, units));
-}
 
 struct Item {
     int32_t r, h0, n0, kbeg, kend, flags, slot, hpw;
@@ -82,23 +49,6 @@ int heads_per_group(int32_t nodes, int32_t kv_heads, int32_t qpk) {
     while (h > 1 && h > kv_heads) h >>= 1;
     return h;
 }
-
-int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
-
-// Cost of one key of a work item in quarter key-steps of a one-head item.  A two-head
-// item stages both heads' K/V but every wave still runs one head's 16 MFMAs per tile,
-// so a tile costs it ~1.25x a one-head tile, not 2x (per-workgroup timestamps: 1.30 vs
-// 1.03 us per tile on the mixed batch of config 5).  Weighting by the head count left
-// two-head chunks at half the length of one-head chunks of the same cost.
-int64_t cost_weight(int hpw) { return hpw == 2 ? 5 : 4; }
-
-// A tree tile takes the general loop (ancestor masks, per-key slot addresses) and costs
-// about two prefix tiles (per-workgroup timestamps on config 2: 16.3 us for the last-chunk
-// items of 64-node trees, 11 prefix tiles + 2 tree tiles, against 13.2 us for 12 prefix
-// tiles).  The chunk lengths of a split prefix are set so that the last chunk, which also
-// walks the tree, ends level with the others: the prefix is cut as if it held this many
-// keys per tree node more, within the same number of chunks.
-constexpr int64_t kTreeKeyWeight = 2;
 
 // MI355X dispatches workgroup i of a launch to XCD i % 8, and each XCD has its own L2.
 // The node blocks of one (request, head group, prefix chunk) stream the same K/V, and
@@ -207,7 +157,13 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
         return fail(TV_ERR_INVALID, "plan: chunk_keys %d must be a non-negative multiple of 32", chunk_keys);
     }
     int32_t max_nodes = 1;
-    int64_t total_cost = 0, units = 0;
+    PlanTotals totals = {};
+    totals.compute_units = num_compute_units;
+    struct Request {
+        int64_t units;   // items of the uncut request
+        int32_t hpw, groups, blocks;
+    };
+    std::vector<Request> shape(num_requests);
     for (int32_t r = 0; r < num_requests; ++r) {
         const int32_t p = prefix_lens_host[r], t = node_counts_host[r];
         if (p < 0) return fail(TV_ERR_INVALID, "plan: negative prefix length for request %d", r);
@@ -217,87 +173,81 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
                         max_tree_nodes);
         }
         max_nodes = std::max(max_nodes, t);
-        const int hpw = heads_per_group(t, num_kv_heads, qpk);
-        const int npw = nodes_per_item(hpw, qpk);
-        const int64_t groups = (num_kv_heads + hpw - 1) / hpw;
-        const int64_t blocks = (t + npw - 1) / npw;
-        units += groups * blocks;
-        total_cost += groups * blocks * cost_weight(hpw) * (static_cast<int64_t>(p) + t);
+        Request& q = shape[r];
+        q.hpw = heads_per_group(t, num_kv_heads, qpk);
+        const int npw = nodes_per_item(q.hpw, qpk);
+        q.groups = (num_kv_heads + q.hpw - 1) / q.hpw;
+        q.blocks = (t + npw - 1) / npw;
+        q.units = static_cast<int64_t>(q.groups) * q.blocks;
+        totals.units += q.units;
+        totals.prefix_cost += q.units * cost_weight(q.hpw) * p;
+        totals.cost += q.units * cost_weight(q.hpw) * (static_cast<int64_t>(p) + t);
     }
-    const int64_t target = std::max<int64_t>(kMinChunkKeys, total_cost / num_compute_units);
+    totals.target = std::max<int64_t>(kMinChunkKeys, totals.cost / num_compute_units);
     if (chunk_keys > max_chunk) {
         return fail(TV_ERR_INVALID, "plan: chunk_keys %d exceeds %lld", chunk_keys, (long long)max_chunk);
     }
 
     // Chunk length of a prefix of p keys before a tree of t nodes (hpw heads per item) for
-    // chunk target `tau` (in cost units): the longest multiple of 32 keys whose cost is not
-    // above tau gives the chunk count; the chunks then share the prefix and the tree's
-    // weight (kTreeKeyWeight keys a node) evenly, in multiples of 32 keys, as far as that
-    // keeps the chunk count (the chunks before the last stay below the prefix) and the cap.
+    // chunk target `tau` (in cost units).
     auto chunk_for = [&](int64_t p, int64_t t, int hpw, int64_t tau) -> int64_t {
-        int64_t chunk = std::min(round_up(std::max<int64_t>(kMinChunkKeys, tau / cost_weight(hpw)), 32), max_chunk);
-        const int64_t nchunks = p > 0 ? (p + chunk - 1) / chunk : 1;
-        chunk = round_up((p + nchunks - 1) / std::max<int64_t>(nchunks, 1), 32);
-        if (nchunks > 1) {
-            const int64_t even = round_up((p + kTreeKeyWeight * t + nchunks - 1) / nchunks, 32);
-            const int64_t keep = std::min((p - 1) / (nchunks - 1) / 32 * 32, max_chunk);
-            chunk = std::max(chunk, std::min(even, keep));
-        }
-        return chunk < 32 ? 32 : chunk;
+        const uint32_t chunks = chunk_count(static_cast<uint32_t>(p), chunk_limit(tau / cost_weight(hpw), max_chunk));
+        return chunk_keys_of(static_cast<uint32_t>(p), static_cast<uint32_t>(t), chunks, max_chunk);
     };
     auto items_for = [&](int64_t tau) -> int64_t {
+        const uint32_t one = chunk_limit(tau / cost_weight(1), max_chunk), two = chunk_limit(tau / cost_weight(2), max_chunk);
         int64_t n = 0;
         for (int32_t r = 0; r < num_requests; ++r) {
-            const int64_t p = prefix_lens_host[r];
-            const int hpw = heads_per_group(node_counts_host[r], num_kv_heads, qpk);
-            const int npw = nodes_per_item(hpw, qpk);
-            const int64_t per = static_cast<int64_t>((num_kv_heads + hpw - 1) / hpw) * ((node_counts_host[r] + npw - 1) / npw);
-            const int64_t chunk = chunk_for(p, node_counts_host[r], hpw, tau);
-            n += per * (p > 0 ? (p + chunk - 1) / chunk : 1);
+            n += shape[r].units * chunk_count(static_cast<uint32_t>(prefix_lens_host[r]), shape[r].hpw == 2 ? two : one);
         }
         return n;
     };
-    int64_t tau = target;
-    const int64_t now = chunk_keys == 0 ? items_for(target) : 0;
-    if (chunk_keys == 0 && now <= kFillRounds * num_compute_units) {
-        // Smallest multiple of kTauStep whose item count is at most `cap`; 0 if an uncut batch has more.
-        auto fit = [&](int64_t cap) -> int64_t {
-            const int64_t most = total_cost / kTauStep + 1;   // uncut
-            int64_t lo = 1, hi = std::max<int64_t>(1, std::min(most, total_cost / cap / kTauStep));
-            while (items_for(hi * kTauStep) > cap) {
-                if (hi >= most) return 0;
-                lo = hi + 1;
-                hi = std::min(most, 2 * hi);
-            }
-            while (lo < hi) {
-                const int64_t mid = lo + (hi - lo) / 2;
-                if (items_for(mid * kTauStep) <= cap) hi = mid; else lo = mid + 1;
-            }
-            return lo * kTauStep;
-        };
-        const int64_t rounds = std::max<int64_t>(1, (now + num_compute_units - 1) / num_compute_units);
-        int64_t best = 0;
-        for (int64_t k = 1; k <= rounds; ++k) {
-            const int64_t cap = k == 1 ? one_round_items(total_cost, units, num_compute_units) : k * num_compute_units;
-            const int64_t t = fit(cap);
-            const int64_t span = k * (t + kRoundCost) + kSlotCost * cap;
-            if (t > 0 && (best == 0 || span < best)) {
-                best = span;
-                tau = t;
-            }
-        }
+    int64_t tau = totals.target;
+    if (chunk_keys == 0) {
+        totals.now = items_for(tau);
+        tau = plan_target(
+            totals, [&](int64_t i, int64_t step, int64_t cap) { return items_for(i * step) <= cap; },
+            [&](int64_t lo, int64_t hi, int64_t step, int64_t cap) {
+                while (lo < hi) {
+                    const int64_t mid = lo + (hi - lo) / 2;
+                    if (items_for(mid * step) <= cap) hi = mid; else lo = mid + 1;
+                }
+                return lo;
+            },
+            [&](int64_t at) {
+                const uint32_t one = chunk_limit(at / cost_weight(1), max_chunk), two = chunk_limit(at / cost_weight(2), max_chunk);
+                PlanSpan all = {0, 0, 0};
+                for (int32_t r = 0; r < num_requests; ++r) {
+                    const int32_t t = node_counts_host[r];
+                    const PlanSpan s = request_span(static_cast<uint32_t>(prefix_lens_host[r]), static_cast<uint32_t>(t),
+                                                    static_cast<int64_t>(t) * qpk * num_kv_heads, cost_weight(shape[r].hpw),
+                                                    shape[r].hpw == 2 ? two : one, max_chunk);
+                    all.longest = std::max(all.longest, s.longest);
+                    all.partial_rows += s.partial_rows;
+                    all.parts = std::max(all.parts, s.parts);
+                }
+                return span_estimate(all);
+            });
     }
 
     std::vector<Item> items;
+    int64_t num_items = 0;
     int32_t num_slots = 0, num_groups = 0;
+    const bool build = items_host || groups_host;   // else the caller asks for the counts
     for (int32_t r = 0; r < num_requests; ++r) {
         const int32_t p = prefix_lens_host[r], t = node_counts_host[r];
-        const int hpw = heads_per_group(t, num_kv_heads, qpk);
-        const int npw = nodes_per_item(hpw, qpk);
-        const int32_t groups = (num_kv_heads + hpw - 1) / hpw;
-        const int32_t blocks = (t + npw - 1) / npw;
+        const int hpw = shape[r].hpw, npw = nodes_per_item(hpw, qpk);
+        const int32_t groups = shape[r].groups, blocks = shape[r].blocks;
         const int64_t chunk = chunk_keys > 0 ? chunk_keys : chunk_for(p, t, hpw, tau);
         const int32_t nchunks = p > 0 ? static_cast<int32_t>((p + chunk - 1) / chunk) : 1;
+        num_items += shape[r].units * nchunks;
+        if (!build) {
+            if (nchunks > 1) {
+                num_slots += static_cast<int32_t>(shape[r].units * nchunks);
+                num_groups += static_cast<int32_t>(shape[r].units);
+            }
+            continue;
+        }
         for (int32_t hg = 0; hg < groups; ++hg) {
             for (int32_t nb = 0; nb < blocks; ++nb) {
                 const int32_t first_slot = nchunks > 1 ? num_slots : -1;
@@ -359,7 +309,7 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
             o[7] = items[i].hpw;
         }
     }
-    info->num_items = static_cast<int32_t>(items.size());
+    info->num_items = static_cast<int32_t>(num_items);
     info->num_groups = num_groups;
     info->num_partial_slots = num_slots;
     info->ancestor_words_per_row = (max_nodes + 63) / 64;

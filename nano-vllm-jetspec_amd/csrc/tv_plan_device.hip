@@ -9,10 +9,10 @@
 //
 // One 1024-thread workgroup (steps 1 and 2 in wave 0 alone, one request per lane and no
 // barrier, for batches of at most 64 requests):
-//   1. per request: KV heads per group, node blocks, cost; the total cost (reduction);
+//   1. per request: KV heads per group, node blocks, cost; the total cost (reduction); the
+//      chunk target (tv_plan_rule.h, the host's);
 //   2. per request: prefix chunk length and count (the host formulas), item / group /
-//      slot counts, and their exclusive prefix sums (one scan); the host's refit of the
-//      chunk target when the last round of items is part-empty;
+//      slot counts, and their exclusive prefix sums (one scan);
 //   3. the items in the host comparator's order, (~cost, request, head group, chunk,
 //      block), longest first: up to 128 requests by ranking each request's two cost
 //      classes (its chunks before the last, its last chunk) and placing every item at its
@@ -28,6 +28,7 @@
 #include <algorithm>
 
 #include "tv_internal.h"
+#include "tv_plan_rule.h"
 
 namespace tv {
 namespace {
@@ -39,10 +40,8 @@ constexpr int kMaxPlanRequests = 2048;
 // XCD placement may park a 16-bit position in bits 48-63.
 static_assert(kMaxPlanRequests <= 65536 && kMaxSortItems <= 65536, "sorted keys pack 16-bit fields");
 constexpr int kMaxPlanNodes = 2048;     // tree nodes of one request (the attention kernel's page-mode cache)
-constexpr int kMinChunkKeys = 64;
 constexpr int kMaxChunkPages = 512;
 constexpr int kXcds = 8;
-constexpr int64_t kFillRounds = 4;
 
 struct PlanArgs {
     const int32_t* prefix_lens;
@@ -57,34 +56,9 @@ struct PlanArgs {
 // Nodes of one KV head per work item and the two-head rule of the host planner (tv_plan.cpp).
 __host__ __device__ __forceinline__ int nodes_per_item(int hpw, int qpk) { return (8 / hpw) * (32 / qpk); }
 
-__device__ __forceinline__ int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
-
-// Cost of one key of a work item in quarter key-steps of a one-head item: a two-head
-// tile costs ~1.25x a one-head tile (each wave still runs one head's MFMAs).  The host
-// planner uses the same weights.
-__device__ __forceinline__ int64_t cost_weight(int hpw) { return hpw == 2 ? 5 : 4; }
-
-// The host planner's choice of the chunk target (tv_plan.cpp gives the reasons and figures).
-constexpr int64_t kPartialCost = 5;
-constexpr int64_t kRoundCost = 1000;
-constexpr int64_t kSlotCost = 2;
-constexpr int64_t kTauStep = 128;
-
-__device__ __forceinline__ int64_t one_round_items(int64_t total_cost, int64_t units, int64_t compute_units) {
-    const int64_t x = total_cost / kPartialCost;
-    int64_t n = compute_units;
-    if (x < compute_units * compute_units) {
-        n = 0;
-        for (int64_t bit = int64_t{1} << 20; bit > 0; bit >>= 1) {   // integer square root
-            if ((n + bit) * (n + bit) <= x) n += bit;
-        }
-    }
-    return min(compute_units, max(n, units));
-}
-
 constexpr int kPlanWaves = kPlanThreads / 64;
 constexpr int kPer = kMaxSortItems / kPlanThreads;   // sorted positions per thread
-constexpr int kProbeWaves = 4;   // waves that probe chunk targets in the refit (one per SIMD)
+constexpr int kProbeWaves = 4;   // waves that probe chunk targets (one per SIMD)
 
 // One lane move of a wave scan (gfx9 DPP, on both halves of an int64): `kCtrl` is row_shr:n
 // (0x110 + n) or a row broadcast, `kRowMask` the rows that receive; a lane with no source, or
@@ -150,6 +124,17 @@ __device__ void block_scan3(int64_t (&v)[3], int waves, int64_t* scratch, int64_
 // Sum over one wave (returned to every lane).
 __device__ __forceinline__ int64_t wave_sum(int64_t v) { return lane_value(wave_inclusive_sum(v), 63); }
 
+// Maximum of non-negative values over one wave (returned to every lane).
+__device__ __forceinline__ int64_t wave_max(int64_t x) {
+    x = max(x, dpp_move<0x111>(x));
+    x = max(x, dpp_move<0x112>(x));
+    x = max(x, dpp_move<0x114>(x));
+    x = max(x, dpp_move<0x118>(x));
+    x = max(x, dpp_move<0x142, 0xa>(x));
+    x = max(x, dpp_move<0x143, 0xc>(x));
+    return lane_value(x, 63);
+}
+
 // Block-wide sum of one int64 per thread, returned to all; as for block_scan3, only the
 // first `waves` waves (wave-uniform, at least 1) may hold nonzero values.
 __device__ int64_t block_sum(int64_t v, int waves, int64_t* scratch) {
@@ -198,23 +183,9 @@ __device__ __forceinline__ int div_small(int a, int b, int& rem) {
 }
 
 // The host planner's chunk length (tv_plan.cpp, chunk_for) for a prefix of p keys before
-// a tree of n nodes, with q = tau / cost_weight(hpw) precomputed: the chunk count from
-// min(round_up(max(64, q), 32), max_chunk), then the prefix and the tree's weight shared
-// evenly over the chunks as far as the count and the cap allow.  Every quantity after the
-// first min is below 2^32.
-constexpr uint32_t kTreeKeyWeight = 2;   // prefix keys a tree node costs (tv_plan.cpp)
-
+// a tree of n nodes, with q = tau / cost_weight(hpw) precomputed.
 __device__ __forceinline__ uint32_t chunk_of(uint32_t p, uint32_t n, int64_t q, int64_t max_chunk) {
-    const int64_t c0 = min(round_up(max(static_cast<int64_t>(kMinChunkKeys), min(q, max_chunk)), 32), max_chunk);
-    const uint32_t c = static_cast<uint32_t>(c0);
-    const uint32_t nchunks = p > 0 ? (p + c - 1) / c : 1;
-    uint32_t chunk = ((p + nchunks - 1) / nchunks + 31) / 32 * 32;
-    if (nchunks > 1) {
-        const uint32_t even = ((p + kTreeKeyWeight * n + nchunks - 1) / nchunks + 31) / 32 * 32;
-        const uint32_t keep = min((p - 1) / (nchunks - 1) / 32 * 32, static_cast<uint32_t>(max_chunk));
-        chunk = max(chunk, min(even, keep));
-    }
-    return chunk < 32 ? 32 : chunk;
+    return chunk_keys_of(p, n, chunk_count(p, chunk_limit(q, max_chunk)), max_chunk);
 }
 
 // Plans in one 1024-thread workgroup.  The prefix lengths and node counts are read once into
@@ -257,14 +228,6 @@ plan_device_kernel(const PlanArgs a) {
         s.NB = bits & 0xfff;
         return s;
     };
-    // Items of request r at chunk target tau (q4 = tau / 4, q5 = tau / 5).
-    auto request_items = [&](int r, int64_t q4, int64_t q5) -> int64_t {
-        const uint32_t p = static_cast<uint32_t>(req_p[r]);
-        const ReqShape s = shape_at(r);
-        const uint32_t chunk = chunk_of(p, static_cast<uint32_t>(req_n[r]), s.hpw == 2 ? q5 : q4, max_chunk);
-        return static_cast<int64_t>(s.G) * s.NB * (p > 0 ? (p + chunk - 1) / chunk : 1u);
-    };
-
     // Step 3's cost classes (ranked there) in stream_id, which the placement overwrites later.
     // Class 0: the chunks before the last (the whole request when both costs are equal), class
     // 1: the last chunk.  An absent class has no items and a cost field above every real one,
@@ -315,7 +278,7 @@ plan_device_kernel(const PlanArgs a) {
         }
         bool bad = false;
         int my_shapes = 0;
-        int64_t my_cost = 0, my_units = 0;
+        int64_t my_cost = 0, my_prefix_cost = 0, my_units = 0;
         for (int r = t; r < R; r += kPlanThreads) {
             const int p = a.prefix_lens[r], n = a.node_counts[r];
             bad |= p < 0 || n < 1 || n > kMaxPlanNodes;
@@ -325,18 +288,105 @@ plan_device_kernel(const PlanArgs a) {
             const ReqShape s = req_shape(nc, KV, NW);
             req_bits[r] = static_cast<uint16_t>(s.NB | (s.hpw == 2 ? 0x8000 : 0));
             my_shapes |= (s.NB > 1 ? 1 : 0) | (s.NB > 1 && s.NB % kXcds ? 2 : 0);
-            my_units += static_cast<int64_t>(s.G) * s.NB;
-            my_cost += static_cast<int64_t>(s.G) * s.NB * cost_weight(s.hpw) * (static_cast<int64_t>(pc) + nc);
+            const int64_t units = static_cast<int64_t>(s.G) * s.NB, weight = units * cost_weight(s.hpw);
+            my_units += units;
+            my_prefix_cost += weight * pc;
+            my_cost += weight * (static_cast<int64_t>(pc) + nc);
         }
         if (!one_wave) __syncthreads();   // the flags are cleared before anyone sets them
         if (bad) atomicOr(&shared_flag, 1);
         if (my_shapes) atomicOr(&shape_flag, my_shapes);
         // The block sum's barriers also publish req_p, req_n, req_bits and the flags.
-        const int64_t total_cost = one_wave ? wave_sum(my_cost)
-                                            : block_sum(my_cost, (min(R, kPlanThreads) + 63) / 64, scan);
-        const int64_t units = one_wave ? wave_sum(my_units)
-                                       : block_sum(my_units, (min(R, kPlanThreads) + 63) / 64, scan);
-        const int64_t target = max(static_cast<int64_t>(kMinChunkKeys), total_cost / a.compute_units);
+        const int waves = (min(R, kPlanThreads) + 63) / 64;
+        PlanTotals all = {};
+        all.compute_units = a.compute_units;
+        all.cost = one_wave ? wave_sum(my_cost) : block_sum(my_cost, waves, scan);
+        all.target = max(static_cast<int64_t>(kMinChunkKeys), all.cost / a.compute_units);
+        int64_t tau = all.target;
+
+        // 1b. The chunk target (plan_target).  Wave 0 alone counts the items of its lanes' requests
+        // and bisects; the block counts in every wave, and one wave per SIMD probes one target each
+        // (a 5-way search, two barriers per step; more probing waves would share the SIMDs and make
+        // every step as much longer).
+        if (a.chunk_keys == 0) {
+            // The lane's requests: one, or every 64th.
+            uint32_t p0 = 0;
+            int64_t units0 = 0;
+            bool two0 = false;
+            if (one_wave && lane < R) {
+                const ReqShape s = shape_at(lane);
+                p0 = static_cast<uint32_t>(req_p[lane]);
+                units0 = static_cast<int64_t>(s.G) * s.NB;
+                two0 = s.hpw == 2;
+            }
+            auto count_at = [&](int64_t target) __attribute__((always_inline)) -> int64_t {
+                const uint32_t one = chunk_limit(target / cost_weight(1), max_chunk);
+                const uint32_t two = chunk_limit(target / cost_weight(2), max_chunk);
+                if (one_wave) return wave_sum(units0 * chunk_count(p0, two0 ? two : one));
+                int64_t n = 0;
+                for (int r = lane; r < R; r += 64) {
+                    const ReqShape s = shape_at(r);
+                    n += static_cast<int64_t>(s.G) * s.NB * chunk_count(static_cast<uint32_t>(req_p[r]), s.hpw == 2 ? two : one);
+                }
+                return wave_sum(n);
+            };
+            // Which of the items at v[k] fit `cap`, bit k, in every thread.
+            auto probe4 = [&](int64_t v0, int64_t v1, int64_t v2, int64_t v3, int64_t cap) -> int {
+                if (wave < kProbeWaves) {
+                    const int64_t v = wave == 0 ? v0 : wave == 1 ? v1 : wave == 2 ? v2 : v3;
+                    const int64_t n = count_at(v);
+                    if (lane == 0) probe_fits[wave] = n <= cap ? 1 : 0;
+                }
+                __syncthreads();
+                int bits = 0;
+#pragma unroll
+                for (int k = 0; k < kProbeWaves; ++k) bits |= probe_fits[k] << k;
+                __syncthreads();   // every thread has read probe_fits
+                return bits;
+            };
+            all.now = count_at(tau);
+            if (all.now <= kFillRounds * all.compute_units) {
+                all.prefix_cost = one_wave ? wave_sum(my_prefix_cost) : block_sum(my_prefix_cost, waves, scan);
+                all.units = one_wave ? wave_sum(my_units) : block_sum(my_units, waves, scan);
+                tau = plan_target(
+                    all, [&](int64_t i, int64_t step, int64_t cap) { return count_at(i * step) <= cap; },
+                    [&](int64_t lo, int64_t hi, int64_t step, int64_t cap) {
+                        while (lo < hi) {
+                            const int64_t span = hi - lo;
+                            if (one_wave) {
+                                const int64_t mid = lo + span / 2;
+                                if (count_at(mid * step) <= cap) hi = mid; else lo = mid + 1;
+                                continue;
+                            }
+                            const int64_t v[4] = {lo + span / 5, lo + span * 2 / 5, lo + span * 3 / 5, lo + span * 4 / 5};
+                            const int bits = probe4(v[0] * step, v[1] * step, v[2] * step, v[3] * step, cap);
+                            int64_t new_lo = lo, new_hi = hi;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) {
+                                if (bits >> k & 1) new_hi = min(new_hi, v[k]); else new_lo = max(new_lo, v[k] + 1);
+                            }
+                            lo = new_lo;
+                            hi = new_hi;
+                        }
+                        return lo;
+                    },
+                    [&](int64_t at) {
+                        const uint32_t one = chunk_limit(at / cost_weight(1), max_chunk);
+                        const uint32_t two = chunk_limit(at / cost_weight(2), max_chunk);
+                        PlanSpan mine = {0, 0, 0};
+                        for (int r = lane; r < R; r += 64) {
+                            const int hpw = (req_bits[r] >> 15) + 1, n = req_n[r];
+                            const PlanSpan s = request_span(static_cast<uint32_t>(req_p[r]), static_cast<uint32_t>(n),
+                                                            static_cast<int64_t>(n) * QPK * KV, cost_weight(hpw),
+                                                            hpw == 2 ? two : one, max_chunk);
+                            mine.longest = max(mine.longest, s.longest);
+                            mine.partial_rows += s.partial_rows;
+                            mine.parts = max(mine.parts, s.parts);
+                        }
+                        return span_estimate({wave_max(mine.longest), wave_sum(mine.partial_rows), wave_max(mine.parts)});
+                    });
+            }
+        }
 
         // 2. Chunking and per-request counts at chunk target tau (or the forced chunk length):
         // chunk lengths and counts per request, their exclusive prefix sums (one scan) and the
@@ -396,95 +446,7 @@ plan_device_kernel(const PlanArgs a) {
             }
             if (!one_wave) __syncthreads();
         };
-        chunking(target);
-
-        // 2b. The host's choice of the chunk target for at most kFillRounds rounds of items, then
-        // the chunking again at it.  The count falls as the target grows, so any search finds the
-        // host's result: wave 0 alone gallops and bisects; the block has one wave per SIMD probe
-        // one target each (a 5-way search, two barriers per step; more probing waves would share
-        // the SIMDs and make every step as much longer).
-        if (a.chunk_keys == 0 && tot[0] <= kFillRounds * a.compute_units) {
-            // Whether the items at v[k] * kTauStep fit `cap`, bit k, in every thread taking part.
-            auto count_at = [&](int64_t i) -> int64_t {
-                const int64_t q4 = i * kTauStep / 4, q5 = i * kTauStep / 5;
-                int64_t n = 0;
-                for (int r = lane; r < R; r += 64) n += request_items(r, q4, q5);
-                return wave_sum(n);
-            };
-            auto probe4 = [&](int64_t v0, int64_t v1, int64_t v2, int64_t v3, int64_t cap) -> int {
-                if (wave < kProbeWaves) {
-                    const int64_t v = wave == 0 ? v0 : wave == 1 ? v1 : wave == 2 ? v2 : v3;
-                    const int64_t n = count_at(v);
-                    if (lane == 0) probe_fits[wave] = n <= cap ? 1 : 0;
-                }
-                __syncthreads();
-                int bits = 0;
-#pragma unroll
-                for (int k = 0; k < kProbeWaves; ++k) bits |= probe_fits[k] << k;
-                __syncthreads();   // every thread has read probe_fits
-                return bits;
-            };
-            const int64_t most = total_cost / kTauStep + 1;   // uncut
-            auto fit = [&](int64_t cap) -> int64_t {
-                int64_t lo = 1, hi = max(int64_t{1}, min(most, total_cost / cap / kTauStep));
-                if (one_wave) {
-                    while (count_at(hi) > cap) {
-                        if (hi >= most) return 0;
-                        lo = hi + 1;
-                        hi = min(most, 2 * hi);
-                    }
-                    while (lo < hi) {
-                        const int64_t mid = lo + (hi - lo) / 2;
-                        if (count_at(mid) <= cap) hi = mid; else lo = mid + 1;
-                    }
-                } else {
-                    for (;;) {
-                        const int64_t v1 = min(most, 2 * hi), v2 = min(most, 4 * hi), v3 = min(most, 8 * hi);
-                        const int bits = probe4(hi, v1, v2, v3, cap);   // fits from some bit on
-                        if (bits & 1) break;
-                        lo = hi + 1;
-                        hi = v1;
-                        if (bits & 2) break;
-                        lo = v1 + 1;
-                        hi = v2;
-                        if (bits & 4) break;
-                        lo = v2 + 1;
-                        hi = v3;
-                        if (bits & 8) break;
-                        if (v3 >= most) return 0;
-                        lo = v3 + 1;
-                        hi = min(most, 2 * v3);
-                    }
-                    while (lo < hi) {
-                        const int64_t span = hi - lo;
-                        const int64_t v0 = lo + span / 5, v1 = lo + span * 2 / 5, v2 = lo + span * 3 / 5,
-                                      v3 = lo + span * 4 / 5;   // in [lo, hi)
-                        const int bits = probe4(v0, v1, v2, v3, cap);
-                        const int64_t v[4] = {v0, v1, v2, v3};
-                        int64_t new_lo = lo, new_hi = hi;
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            if (bits >> k & 1) new_hi = min(new_hi, v[k]); else new_lo = max(new_lo, v[k] + 1);
-                        }
-                        lo = new_lo;
-                        hi = new_hi;
-                    }
-                }
-                return lo * kTauStep;
-            };
-            const int64_t rounds = max(int64_t{1}, (tot[0] + a.compute_units - 1) / a.compute_units);
-            int64_t best = 0, tau = target;
-            for (int64_t k = 1; k <= rounds; ++k) {
-                const int64_t cap = k == 1 ? one_round_items(total_cost, units, a.compute_units) : k * a.compute_units;
-                const int64_t found = fit(cap);
-                const int64_t span = k * (found + kRoundCost) + kSlotCost * cap;
-                if (found > 0 && (best == 0 || span < best)) {
-                    best = span;
-                    tau = found;
-                }
-            }
-            if (tau != target) chunking(tau);
-        }
+        chunking(tau);
         if (one_wave && lane < R) write_classes(lane);
     }
     __syncthreads();
