@@ -191,43 +191,50 @@ int plan(const int32_t* prefix_lens_host, const int32_t* node_counts_host, int32
     // Chunk length of a prefix of p keys before a tree of t nodes (hpw heads per item) for
     // chunk target `tau` (in cost units).
     auto chunk_for = [&](int64_t p, int64_t t, int hpw, int64_t tau) -> int64_t {
-        const uint32_t chunks = chunk_count(static_cast<uint32_t>(p), chunk_limit(tau / cost_weight(hpw), max_chunk));
+        const uint32_t chunks = chunk_count(static_cast<uint32_t>(p), chunk_limit(tau, hpw, max_chunk));
         return chunk_keys_of(static_cast<uint32_t>(p), static_cast<uint32_t>(t), chunks, max_chunk);
     };
     auto items_for = [&](int64_t tau) -> int64_t {
-        const uint32_t one = chunk_limit(tau / cost_weight(1), max_chunk), two = chunk_limit(tau / cost_weight(2), max_chunk);
+        const uint32_t one = chunk_limit(tau, 1, max_chunk), two = chunk_limit(tau, 2, max_chunk);
         int64_t n = 0;
         for (int32_t r = 0; r < num_requests; ++r) {
             n += shape[r].units * chunk_count(static_cast<uint32_t>(prefix_lens_host[r]), shape[r].hpw == 2 ? two : one);
         }
         return n;
     };
+    auto span_at = [&](int64_t at) {
+        const uint32_t one = chunk_limit(at, 1, max_chunk), two = chunk_limit(at, 2, max_chunk);
+        PlanSpan all = {0, 0, 0};
+        for (int32_t r = 0; r < num_requests; ++r) {
+            const int32_t t = node_counts_host[r];
+            const PlanSpan s = request_span(static_cast<uint32_t>(prefix_lens_host[r]), static_cast<uint32_t>(t),
+                                            static_cast<int64_t>(t) * qpk * num_kv_heads, cost_weight(shape[r].hpw),
+                                            shape[r].hpw == 2 ? two : one, max_chunk);
+            all.longest = std::max(all.longest, s.longest);
+            all.partial_rows += s.partial_rows;
+            all.parts = std::max(all.parts, s.parts);
+        }
+        return all;
+    };
     int64_t tau = totals.target;
     if (chunk_keys == 0) {
         totals.now = items_for(tau);
         tau = plan_target(
-            totals, [&](int64_t i, int64_t step, int64_t cap) { return items_for(i * step) <= cap; },
-            [&](int64_t lo, int64_t hi, int64_t step, int64_t cap) {
-                while (lo < hi) {
-                    const int64_t mid = lo + (hi - lo) / 2;
-                    if (items_for(mid * step) <= cap) hi = mid; else lo = mid + 1;
+            totals,
+            [&](int64_t lo, int64_t hi, int64_t guess, bool sure, int64_t step, int64_t cap) -> int64_t {
+                while (lo < hi || !sure) {
+                    if (items_for(guess * step) <= cap) {
+                        hi = guess;
+                        sure = true;
+                    } else {
+                        if (guess == hi) return 0;
+                        lo = guess + 1;
+                    }
+                    guess = lo + (hi - lo) / 2;
                 }
                 return lo;
             },
-            [&](int64_t at) {
-                const uint32_t one = chunk_limit(at / cost_weight(1), max_chunk), two = chunk_limit(at / cost_weight(2), max_chunk);
-                PlanSpan all = {0, 0, 0};
-                for (int32_t r = 0; r < num_requests; ++r) {
-                    const int32_t t = node_counts_host[r];
-                    const PlanSpan s = request_span(static_cast<uint32_t>(prefix_lens_host[r]), static_cast<uint32_t>(t),
-                                                    static_cast<int64_t>(t) * qpk * num_kv_heads, cost_weight(shape[r].hpw),
-                                                    shape[r].hpw == 2 ? two : one, max_chunk);
-                    all.longest = std::max(all.longest, s.longest);
-                    all.partial_rows += s.partial_rows;
-                    all.parts = std::max(all.parts, s.parts);
-                }
-                return span_estimate(all);
-            });
+            [&](int64_t at, int64_t base) { return gains(span_at(at), span_at(base)); });
     }
 
     std::vector<Item> items;

@@ -124,15 +124,22 @@ __device__ void block_scan3(int64_t (&v)[3], int waves, int64_t* scratch, int64_
 // Sum over one wave (returned to every lane).
 __device__ __forceinline__ int64_t wave_sum(int64_t v) { return lane_value(wave_inclusive_sum(v), 63); }
 
-// Maximum of non-negative values over one wave (returned to every lane).
-__device__ __forceinline__ int64_t wave_max(int64_t x) {
+// Sum and maximum (of non-negative values) over each half of a wave, in its last lane.
+__device__ __forceinline__ int64_t half_sum(int64_t x) {
+    x += dpp_move<0x111>(x);
+    x += dpp_move<0x112>(x);
+    x += dpp_move<0x114>(x);
+    x += dpp_move<0x118>(x);
+    x += dpp_move<0x142, 0xa>(x);   // row_bcast:15
+    return x;
+}
+__device__ __forceinline__ int64_t half_max(int64_t x) {
     x = max(x, dpp_move<0x111>(x));
     x = max(x, dpp_move<0x112>(x));
     x = max(x, dpp_move<0x114>(x));
     x = max(x, dpp_move<0x118>(x));
     x = max(x, dpp_move<0x142, 0xa>(x));
-    x = max(x, dpp_move<0x143, 0xc>(x));
-    return lane_value(x, 63);
+    return x;
 }
 
 // Block-wide sum of one int64 per thread, returned to all; as for block_scan3, only the
@@ -180,12 +187,6 @@ __device__ __forceinline__ int div_small(int a, int b, int& rem) {
     }
     rem = r;
     return q;
-}
-
-// The host planner's chunk length (tv_plan.cpp, chunk_for) for a prefix of p keys before
-// a tree of n nodes, with q = tau / cost_weight(hpw) precomputed.
-__device__ __forceinline__ uint32_t chunk_of(uint32_t p, uint32_t n, int64_t q, int64_t max_chunk) {
-    return chunk_keys_of(p, n, chunk_count(p, chunk_limit(q, max_chunk)), max_chunk);
 }
 
 // Plans in one 1024-thread workgroup.  The prefix lengths and node counts are read once into
@@ -320,8 +321,8 @@ plan_device_kernel(const PlanArgs a) {
                 two0 = s.hpw == 2;
             }
             auto count_at = [&](int64_t target) __attribute__((always_inline)) -> int64_t {
-                const uint32_t one = chunk_limit(target / cost_weight(1), max_chunk);
-                const uint32_t two = chunk_limit(target / cost_weight(2), max_chunk);
+                const uint32_t one = chunk_limit(target, 1, max_chunk);
+                const uint32_t two = chunk_limit(target, 2, max_chunk);
                 if (one_wave) return wave_sum(units0 * chunk_count(p0, two0 ? two : one));
                 int64_t n = 0;
                 for (int r = lane; r < R; r += 64) {
@@ -349,15 +350,22 @@ plan_device_kernel(const PlanArgs a) {
                 all.prefix_cost = one_wave ? wave_sum(my_prefix_cost) : block_sum(my_prefix_cost, waves, scan);
                 all.units = one_wave ? wave_sum(my_units) : block_sum(my_units, waves, scan);
                 tau = plan_target(
-                    all, [&](int64_t i, int64_t step, int64_t cap) { return count_at(i * step) <= cap; },
-                    [&](int64_t lo, int64_t hi, int64_t step, int64_t cap) {
-                        while (lo < hi) {
-                            const int64_t span = hi - lo;
-                            if (one_wave) {
-                                const int64_t mid = lo + span / 2;
-                                if (count_at(mid * step) <= cap) hi = mid; else lo = mid + 1;
+                    all,
+                    [&](int64_t lo, int64_t hi, int64_t guess, bool sure, int64_t step, int64_t cap) -> int64_t {
+                        // One count per step in wave 0; in the block one for the guess, then 5-way.
+                        while (lo < hi || !sure) {
+                            if (one_wave || !sure) {
+                                if (count_at(guess * step) <= cap) {
+                                    hi = guess;
+                                    sure = true;
+                                } else {
+                                    if (guess == hi) return 0;
+                                    lo = guess + 1;
+                                }
+                                guess = lo + (hi - lo) / 2;
                                 continue;
                             }
+                            const int64_t span = hi - lo;
                             const int64_t v[4] = {lo + span / 5, lo + span * 2 / 5, lo + span * 3 / 5, lo + span * 4 / 5};
                             const int bits = probe4(v[0] * step, v[1] * step, v[2] * step, v[3] * step, cap);
                             int64_t new_lo = lo, new_hi = hi;
@@ -370,20 +378,40 @@ plan_device_kernel(const PlanArgs a) {
                         }
                         return lo;
                     },
-                    [&](int64_t at) {
-                        const uint32_t one = chunk_limit(at / cost_weight(1), max_chunk);
-                        const uint32_t two = chunk_limit(at / cost_weight(2), max_chunk);
-                        PlanSpan mine = {0, 0, 0};
-                        for (int r = lane; r < R; r += 64) {
-                            const int hpw = (req_bits[r] >> 15) + 1, n = req_n[r];
-                            const PlanSpan s = request_span(static_cast<uint32_t>(req_p[r]), static_cast<uint32_t>(n),
-                                                            static_cast<int64_t>(n) * QPK * KV, cost_weight(hpw),
-                                                            hpw == 2 ? two : one, max_chunk);
-                            mine.longest = max(mine.longest, s.longest);
-                            mine.partial_rows += s.partial_rows;
-                            mine.parts = max(mine.parts, s.parts);
+                    [&](int64_t at, int64_t base) {
+                        // Up to 32 requests: one plan in each half of the wave.
+                        const bool halves = R <= 32;
+                        PlanSpan whole[2];
+#pragma unroll
+                        for (int pass = 0; pass < 2; ++pass) {
+                            if (halves && pass == 1) break;
+                            const int64_t tau_here = halves ? (lane < 32 ? at : base) : (pass == 0 ? at : base);
+                            const uint32_t one = chunk_limit(tau_here, 1, max_chunk);
+                            const uint32_t two = chunk_limit(tau_here, 2, max_chunk);
+                            PlanSpan mine = {0, 0, 0};
+                            for (int r = halves ? lane & 31 : lane; r < R; r += 64) {
+                                const int hpw = (req_bits[r] >> 15) + 1, n = req_n[r];
+                                const PlanSpan s = request_span(static_cast<uint32_t>(req_p[r]), static_cast<uint32_t>(n),
+                                                                static_cast<int64_t>(n) * QPK * KV, cost_weight(hpw),
+                                                                hpw == 2 ? two : one, max_chunk);
+                                mine.longest = max(mine.longest, s.longest);
+                                mine.partial_rows += s.partial_rows;
+                                mine.parts = max(mine.parts, s.parts);
+                            }
+                            const PlanSpan scan = {half_max(mine.longest), half_sum(mine.partial_rows), half_max(mine.parts)};
+                            const PlanSpan low = {lane_value(scan.longest, 31), lane_value(scan.partial_rows, 31),
+                                                  lane_value(scan.parts, 31)};
+                            const PlanSpan high = {lane_value(scan.longest, 63), lane_value(scan.partial_rows, 63),
+                                                   lane_value(scan.parts, 63)};
+                            if (halves) {
+                                whole[0] = low;
+                                whole[1] = high;
+                            } else {
+                                whole[pass] = {max(low.longest, high.longest), low.partial_rows + high.partial_rows,
+                                               max(low.parts, high.parts)};
+                            }
                         }
-                        return span_estimate({wave_max(mine.longest), wave_sum(mine.partial_rows), wave_max(mine.parts)});
+                        return gains(whole[0], whole[1]);
                     });
             }
         }
@@ -397,14 +425,15 @@ plan_device_kernel(const PlanArgs a) {
         int64_t tot[3];
         auto chunking = [&](int64_t tau) {
             int64_t base[3] = {0, 0, 0};   // items, groups, slots
-            const int64_t q4 = tau / 4, q5 = tau / 5;
+            const uint32_t one = chunk_limit(tau, 1, max_chunk), two = chunk_limit(tau, 2, max_chunk);
             for (int r = r0; r < r1; ++r) {
                 const uint32_t p = static_cast<uint32_t>(req_p[r]);
                 const ReqShape s = shape_at(r);
-                const uint32_t chunk = a.chunk_keys > 0 ? static_cast<uint32_t>(a.chunk_keys)
-                                                        : chunk_of(p, static_cast<uint32_t>(req_n[r]),
-                                                                   s.hpw == 2 ? q5 : q4, max_chunk);
-                const uint32_t nchunks = p > 0 ? (p + chunk - 1) / chunk : 1u;
+                const uint32_t chunk = a.chunk_keys > 0
+                                           ? static_cast<uint32_t>(a.chunk_keys)
+                                           : chunk_keys_of(p, static_cast<uint32_t>(req_n[r]),
+                                                           chunk_count(p, s.hpw == 2 ? two : one), max_chunk);
+                const uint32_t nchunks = p > 0 ? divide(p + chunk - 1, chunk) : 1u;
                 req_chunk[r] = static_cast<int32_t>(chunk);
                 req_nchunks[r] = static_cast<int32_t>(nchunks);
                 const int64_t units = static_cast<int64_t>(s.G) * s.NB;

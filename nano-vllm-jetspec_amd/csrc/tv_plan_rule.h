@@ -32,25 +32,49 @@ constexpr int64_t kTreeKeyWeight = 2;
 
 __host__ __device__ __forceinline__ constexpr int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-// Longest chunk of a request within `quota` keys (the target over its cost weight): it gives
-// the chunk count, ceil(prefix / it); the chunks then share the prefix evenly.
-__host__ __device__ __forceinline__ uint32_t chunk_limit(int64_t quota, int64_t max_chunk) {
-    const int64_t c = quota < max_chunk ? quota : max_chunk;
-    const int64_t r = round_up(c > kMinChunkKeys ? c : kMinChunkKeys, 32);
-    return static_cast<uint32_t>(r < max_chunk ? r : max_chunk);
+// a / b.  A generic 32-bit division is ~35 dependent instructions on the device, and the device
+// planner is one wave's chain of them: below 2^22 a reciprocal's estimate is off by at most one.
+__host__ __device__ __forceinline__ uint32_t divide(uint32_t a, uint32_t b) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if (a < (1u << 22)) {
+        const uint32_t q = static_cast<uint32_t>(static_cast<float>(a) * __builtin_amdgcn_rcpf(static_cast<float>(b)));
+        const int32_t r = static_cast<int32_t>(a - q * b);
+        return r < 0 ? q - 1 : static_cast<uint32_t>(r) >= b ? q + 1 : q;
+    }
+#endif
+    return a / b;
+}
+
+__host__ __device__ __forceinline__ float reciprocal(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_rcpf(x);
+#else
+    return 1.f / x;
+#endif
+}
+
+// Longest chunk of a request whose items may cost `tau` (two heads an item or one): it gives the
+// chunk count, ceil(prefix / it); the chunks then share the prefix evenly.
+__host__ __device__ __forceinline__ uint32_t chunk_limit(int64_t tau, int hpw, int64_t max_chunk) {
+    const uint32_t t = tau < 0xffffffffll ? static_cast<uint32_t>(tau) : 0xffffffffu;
+    const uint32_t quota = hpw == 2 ? t / 5 : t / 4, cap = static_cast<uint32_t>(max_chunk);
+    static_assert(cost_weight(1) == 4 && cost_weight(2) == 5, "the divisors");
+    const uint32_t c = quota < cap ? quota : cap;
+    const uint32_t r = ((c > kMinChunkKeys ? c : kMinChunkKeys) + 31u) / 32u * 32u;
+    return r < cap ? r : cap;
 }
 __host__ __device__ __forceinline__ uint32_t chunk_count(uint32_t prefix, uint32_t limit) {
-    return prefix > 0 ? (prefix + limit - 1) / limit : 1u;
+    return prefix > 0 ? divide(prefix + limit - 1, limit) : 1u;
 }
 
 // Keys of a chunk of a prefix of p keys before a tree of n nodes, cut into `chunks`: the prefix and
 // the tree's weight shared evenly, in multiples of 32 keys, as far as that keeps the count (the
 // chunks before the last stay below the prefix) and the cap.
 __host__ __device__ __forceinline__ uint32_t chunk_keys_of(uint32_t p, uint32_t n, uint32_t chunks, int64_t max_chunk) {
-    uint32_t chunk = ((p + chunks - 1) / chunks + 31) / 32 * 32;
+    uint32_t chunk = (divide(p + chunks - 1, chunks) + 31) / 32 * 32;
     if (chunks > 1) {
-        const uint32_t even = ((p + static_cast<uint32_t>(kTreeKeyWeight) * n + chunks - 1) / chunks + 31) / 32 * 32;
-        const uint32_t keep = (p - 1) / (chunks - 1) / 32 * 32, cap = static_cast<uint32_t>(max_chunk);
+        const uint32_t even = (divide(p + static_cast<uint32_t>(kTreeKeyWeight) * n + chunks - 1, chunks) + 31) / 32 * 32;
+        const uint32_t keep = divide(p - 1, chunks - 1) / 32 * 32, cap = static_cast<uint32_t>(max_chunk);
         const uint32_t level = even < keep ? even : keep;
         const uint32_t most = level < cap ? level : cap;
         chunk = chunk > most ? chunk : most;
@@ -77,10 +101,11 @@ __host__ __device__ __forceinline__ uint32_t chunk_keys_of(uint32_t p, uint32_t 
 // balance without the estimate: 0.934, 50 and 18; never taking it: 0.947, 3 and 2, but half as
 // long again on some that it gains.  The planner does not know the head size, whose partial rows
 // cost from half (64) to four times (256) as much: that is what is left.
-// `fits(i, step, cap)`: whether the items at target i * step number at most cap;
-// `smallest(lo, hi, step, cap)`: the smallest such i in [lo, hi], hi being one; `estimate(tau)`:
-// span_estimate.  Item counts fall as the target grows (chunk_count(p, chunk_limit(q)) does, and
-// the even sharing keeps it), so any search finds the same target.
+// `search(lo, hi, guess, sure, step, cap)`: the smallest i in [lo, hi] whose items at target
+// i * step number at most cap, 0 if hi's do not (`sure`: they do); `guess` is a likely upper bound
+// of it.  `shorter(tau, base)`: gains() of their spans.  Item counts fall as the target grows
+// (chunk_count(p, chunk_limit(q)) does, and the even sharing keeps it), so any search finds the
+// same target.
 constexpr int64_t kRoundCost = 1000;
 constexpr int64_t kSlotCost = 2;
 constexpr int64_t kTauStep = 128;      // 32 keys of a one-head item
@@ -97,6 +122,9 @@ struct PlanSpan {
 };
 __host__ __device__ __forceinline__ int64_t span_estimate(const PlanSpan& s) {
     return kLaunchCost + s.longest + kPartialCost * s.partial_rows / 256 + kPartCost * s.parts;
+}
+__host__ __device__ __forceinline__ bool gains(const PlanSpan& s, const PlanSpan& base) {
+    return span_estimate(s) * (100 + kGainPercent) < span_estimate(base) * 100;
 }
 // A request's share of it: p keys, n nodes, `rows` score rows (over all heads).
 __host__ __device__ __forceinline__ PlanSpan request_span(uint32_t p, uint32_t n, int64_t rows, int64_t weight,
@@ -116,64 +144,55 @@ struct PlanTotals {
     int64_t compute_units;
 };
 
-template <class Fits, class Smallest, class Estimate>
-__host__ __device__ __forceinline__ int64_t plan_target(const PlanTotals& t, Fits fits, Smallest smallest,
-                                                        Estimate estimate) {
+template <class Search, class Shorter>
+__host__ __device__ __forceinline__ int64_t plan_target(const PlanTotals& t, Search search, Shorter shorter) {
     if (t.now > kFillRounds * t.compute_units) return t.target;
-    // A limit is at most quota + 63 keys, and 5 is the largest weight: fewer than `cap` items take a
-    // target above prefix_cost / cap - 315; and one of prefix_cost / (cap - units) + 5 is enough
-    // unless a limit is capped.
-    auto least = [&](int64_t cap) {
-        const int64_t x = static_cast<int64_t>(static_cast<float>(t.prefix_cost) / static_cast<float>(cap) * 0.999998f) - 316;
-        return x > 1 ? x : 1;
-    };
-    const int64_t most = t.cost / kTauStep + 1;   // uncut
-    // The smallest multiple of kTauStep above the even share whose items number at most `cap`, 0 if
-    // there is none.
-    auto fewer = [&](int64_t cap) -> int64_t {
-        if (t.units > cap) return 0;
-        int64_t lo = t.target / kTauStep + 1;
-        const int64_t bound = least(cap) / kTauStep;
-        if (bound > lo) lo = bound;
-        int64_t hi = most;
-        if (t.units < cap) {
-            const float x = static_cast<float>(t.prefix_cost) / static_cast<float>(cap - t.units) * 1.000002f;
-            const int64_t enough = (static_cast<int64_t>(x) + 6) / kTauStep + 1;
-            if (enough < hi) hi = enough;
-        }
-        if (hi < lo) hi = lo;
-        while (!fits(hi, kTauStep, cap)) {
-            if (hi >= most) return 0;   // capped limits
-            lo = hi + 1;
-            hi = 2 * hi < most ? 2 * hi : most;
-            if (hi < lo) hi = lo;
-        }
-        return smallest(lo, hi, kTauStep, cap) * kTauStep;
-    };
-    if (t.now <= t.compute_units) {
-        const int64_t x = t.cost / kItemCost;
-        int64_t n = static_cast<int64_t>(sqrtf(static_cast<float>(x < (int64_t{1} << 40) ? x : (int64_t{1} << 40))));
+    const bool one_round = t.now <= t.compute_units;
+    int64_t balance = 0;
+    if (one_round) {
+        // An integer square root, as far as it matters.
+        if (t.cost >= kItemCost * t.now * t.now || t.units >= t.now || t.cost > INT32_MAX) return t.target;
+        const int32_t x = static_cast<int32_t>(t.cost) / static_cast<int32_t>(kItemCost);
+        int32_t n = static_cast<int32_t>(sqrtf(static_cast<float>(x)));
         while (n * n > x) --n;
-        while ((n + 1) * (n + 1) <= x && n < t.now) ++n;
-        if (n < t.units) n = t.units;
-        if (n >= t.now) return t.target;
-        const int64_t tau = fewer(n);
-        if (tau == 0) return t.target;
-        return estimate(tau) * (100 + kGainPercent) < estimate(t.target) * 100 ? tau : t.target;
+        while ((n + 1) * (n + 1) <= x) ++n;
+        balance = n < t.units ? t.units : n;
     }
+    const float prefix_cost = static_cast<float>(t.prefix_cost);
+    const int64_t most = t.cost / kTauStep + 1;   // uncut
     const int64_t rounds = (t.now + t.compute_units - 1) / t.compute_units;
-    const int64_t cap = rounds * t.compute_units;
-    int64_t best = t.target;
-    if (t.now < cap) {
-        const int64_t lo = least(cap);
-        best = smallest(lo < t.target ? lo : t.target, t.target, 1, cap);
-    }
-    int64_t span = rounds * (best + kRoundCost) + kSlotCost * cap;
-    for (int64_t k = rounds - 1; k >= 1; --k) {
-        const int64_t tau = fewer(k * t.compute_units);
-        if (tau == 0) break;   // fewer rounds hold it no more
-        const int64_t s = k * (tau + kRoundCost) + kSlotCost * k * t.compute_units;
-        if (s < span) {
+    int64_t best = t.target, span = 0;
+    for (int64_t k = rounds; k >= 1; --k) {
+        const int64_t cap = one_round ? balance : k * t.compute_units;
+        const bool refill = !one_round && k == rounds;   // at most the even share; else above it
+        int64_t tau = t.target;
+        if (!refill || t.now < cap) {
+            if (t.units > cap) break;
+            // A limit is at most quota + 63 keys, and 5 is the largest weight: fewer than `cap` items take
+            // a target above prefix_cost / cap - 315, and prefix_cost / (cap - units) + 5 is enough unless
+            // a limit is capped.  Floats, with a margin: bounds only shorten the search.
+            const int64_t step = refill ? 1 : kTauStep;
+            const float above = prefix_cost * reciprocal(static_cast<float>(static_cast<int32_t>(cap))) * 0.99999f;
+            int64_t lo = (static_cast<int32_t>(above < 1e9f ? above : 1e9f) - 316) / step, hi = refill ? t.target : most;
+            const int64_t least = refill ? 1 : t.target / kTauStep + 1;
+            if (lo < least) lo = least;
+            if (hi < lo) {
+                if (refill) lo = hi; else hi = lo;
+            }
+            int64_t guess = hi;
+            if (t.units < cap) {
+                const float enough = prefix_cost * reciprocal(static_cast<float>(static_cast<int32_t>(cap - t.units))) * 1.00001f;
+                guess = (static_cast<int32_t>(enough < 1e9f ? enough : 1e9f) + 6) / step + 1;
+            }
+            if (guess < lo) guess = lo;
+            if (guess > hi) guess = hi;
+            const int64_t found = search(lo, hi, guess, refill, step, cap);
+            if (found == 0) break;   // capped limits: no target holds it
+            tau = found * step;
+        }
+        if (one_round) return shorter(tau, t.target) ? tau : t.target;
+        const int64_t s = k * (tau + kRoundCost) + kSlotCost * cap;
+        if (k == rounds || s < span) {
             span = s;
             best = tau;
         }
