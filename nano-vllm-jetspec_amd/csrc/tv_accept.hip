@@ -16,6 +16,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "tv_internal.h"
 
 namespace tv {
@@ -307,17 +309,19 @@ struct EosIds {
     int64_t held[TV_MAX_HOST_EOS];
 };
 
+template <bool HELD>
 __device__ __forceinline__ bool is_eos(const EosIds& eos, int64_t value) {
     bool hit = false;
-    if (eos.device) {
-        for (int32_t e = 0; e < eos.count; ++e) hit = hit || value == eos.device[e];
-    } else {
+    if constexpr (HELD) {
 #pragma unroll
         for (int32_t e = 0; e < TV_MAX_HOST_EOS; ++e) hit = hit || (e < eos.count && value == eos.held[e]);
+    } else {
+        for (int32_t e = 0; e < eos.count; ++e) hit = hit || value == eos.device[e];
     }
     return hit;
 }
 
+template <bool HELD>
 __global__ void __launch_bounds__(kTruncThreads)
 truncate_accepted_kernel(const int32_t* __restrict__ paths, int32_t stride, const int32_t* __restrict__ lengths,
                          const int64_t* __restrict__ corrections, const void* __restrict__ tokens, int tokens64,
@@ -352,7 +356,7 @@ truncate_accepted_kernel(const int32_t* __restrict__ paths, int32_t stride, cons
                 if (!ignore_eos[r]) {
                     for (int32_t j = 0; j < limit; ++j) {
                         const int64_t v = value(j);
-                        if (is_eos(eos, v)) {
+                        if (is_eos<HELD>(eos, v)) {
                             limit = j + 1;
                             break;
                         }
@@ -383,15 +387,15 @@ truncate_accepted_kernel(const int32_t* __restrict__ paths, int32_t stride, cons
     if (t == 0) commit_offsets[num_requests] = carry;
 }
 
-// The same cut for short paths and up to kTeamMaxRequests requests: a team of lanes per
-// request, one lane per value, so that a request costs one chain of loads (lengths and path,
-// then the token) and not one per path node, which is what bounds so small a kernel: 64
-// requests with 16-entry path rows 12.5 -> 4.3 us.  Every wave scans a pass's limits itself,
-// from LDS.
+// The same cut for short paths and few requests: a team of lanes per request, one lane per
+// value, so that a request costs one chain of loads (lengths and path, then the token) and not
+// one per path node, which is what bounds so small a kernel: 64 requests with 16-entry path rows
+// 8.8 -> 3.4 us.  Every wave scans a pass's limits itself, from LDS.
 constexpr int kTeamMinLanes = 16;   // a pass then holds at most 64 requests, one lane each in the scan
 constexpr int kTeamMaxLanes = 64;
-constexpr int kTeamMaxRequests = 256;
+constexpr int kTeamMinPasses = 2, kTeamMaxPasses = 6;
 
+template <bool HELD>
 __global__ void __launch_bounds__(kTruncThreads)
 truncate_teams_kernel(const int32_t* __restrict__ paths, int32_t stride, int32_t team_shift,
                       const int32_t* __restrict__ lengths, const int64_t* __restrict__ corrections,
@@ -433,7 +437,7 @@ truncate_teams_kernel(const int32_t* __restrict__ paths, int32_t stride, int32_t
                     value = tokens64 ? static_cast<const int64_t*>(tokens)[row]
                                      : static_cast<int64_t>(static_cast<const int32_t*>(tokens)[row]);
                 }
-                const uint64_t ends = __ballot(wanted && j < limit && is_eos(eos, value)) & members;
+                const uint64_t ends = __ballot(wanted && j < limit && is_eos<HELD>(eos, value)) & members;
                 if (ends) limit = __builtin_ctzll(ends) - first + 1;
             }
             if (j == 0) limits[r] = limit;
@@ -476,22 +480,29 @@ int truncate_accepted(const int32_t* paths, int32_t path_stride, const int32_t* 
         !emitted || !commit_paths || !commit_offsets) {
         return fail(TV_ERR_INVALID, "truncate_accepted: null pointer");
     }
-    // A team of 16 to 64 lanes per request up to 256 requests: a pass of 64 requests adds 2.5 us
-    // (64, 128, 256 requests 4.3, 6.9, 11.8 us; a thread per request 12.5, 13.4, 14.9).  Above, or
-    // for longer paths, a thread per request, which takes 1024 requests in one pass.
-    if (path_stride <= kTeamMaxLanes && num_requests <= kTeamMaxRequests) {
-        int32_t shift = 4;
-        while ((1 << shift) < path_stride) ++shift;
+    // A pass takes 64 requests with paths of up to 16 entries, 32 up to 32 and 16 up to 64, and adds
+    // 1.6 us to a launch's 1.8; a thread per request takes 1024 in one pass whose time follows the
+    // longest accepted path: 4.8 us for paths of one node, 6.0 at 8 entries (accepted to a third), 9.9
+    // at 16, 13.4 at 24, 31 at 64.  So two passes (4.9 us) up to 11 entries, then one for every four
+    // entries, and six (11.3) at most, which a longest path of nine nodes repays.  256 requests: 8
+    // entries (four passes) 8.0 against 6.0, 16 entries 8.1 against 9.9, 17 entries (eight) 14.4
+    // against 9.7; 65 of 64 entries (five) 9.3 against 28.
+    int32_t shift = 4;
+    while ((1 << shift) < path_stride && shift < 6) ++shift;
+    const int32_t passes = std::min(kTeamMaxPasses, std::max(kTeamMinPasses, path_stride / 4));
+    const int32_t most = passes * (kTruncThreads >> shift);
+    if (path_stride <= kTeamMaxLanes && num_requests <= most) {
         static_assert(kTeamMinLanes == 1 << 4 && kTruncThreads / kTeamMinLanes <= 64, "one lane per team in the scan");
-        hipLaunchKernelGGL(truncate_teams_kernel, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths,
-                           path_stride, shift, lengths, corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0,
-                           cu_seqlens, num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths,
-                           commit_offsets, status);
+        const auto teams = eos.device ? truncate_teams_kernel<false> : truncate_teams_kernel<true>;
+        hipLaunchKernelGGL(teams, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths, path_stride, shift,
+                           lengths, corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0, cu_seqlens, num_requests,
+                           budgets, ignore_eos, eos, limits, emitted, commit_paths, commit_offsets, status);
         return check_launch("truncate_accepted");
     }
-    hipLaunchKernelGGL(truncate_accepted_kernel, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths,
-                       path_stride, lengths, corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0, cu_seqlens,
-                       num_requests, budgets, ignore_eos, eos, limits, emitted, commit_paths, commit_offsets, status);
+    const auto threads = eos.device ? truncate_accepted_kernel<false> : truncate_accepted_kernel<true>;
+    hipLaunchKernelGGL(threads, dim3(1), dim3(kTruncThreads), 0, as_stream(stream), paths, path_stride, lengths,
+                       corrections, token_ids, tokens_is_int64 != 0 ? 1 : 0, cu_seqlens, num_requests, budgets,
+                       ignore_eos, eos, limits, emitted, commit_paths, commit_offsets, status);
     return check_launch("truncate_accepted");
 }
 }  // namespace
