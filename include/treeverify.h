@@ -513,10 +513,11 @@ int64_t tv_tree_attention_workspace_bytes(int32_t num_partial_slots, int32_t hea
  * out[q, h, :] = sum_k p_k V[k, h/G, :] / sum_k p_k with p_k = exp(s_k - max s) and
  * s_k = scale * q[q,h,:] . K[k, h/G, :] (+ qq_bias[bias_off[r] + local * T + j] for tree
  * key j); key position pos of request r is visible iff pos <= P + local.  Products are exact
- * with fp32 sums, probabilities and the online softmax fp32.  No plan or workspace: a
- * workgroup per 32 score rows of a request and KV head, reading every metadata value from
- * device memory, so the launch is graph-capturable as is.  Out-of-range pages or slots set TV_STATUS_BAD_PAGE and
- * that key is skipped; a row naming a nonexistent request sets TV_STATUS_BAD_REQUEST.
+ * with fp32 sums, probabilities and the online softmax fp32 (f16 operands: a probability enters
+ * the product to 2^-39 of its row's reference).  No plan or workspace: a workgroup per 32 score
+ * rows of a request and KV head (per 4 packed rows for short requests), reading every metadata
+ * value from device memory, so the launch is graph-capturable as is.  Out-of-range pages or slots
+ * set TV_STATUS_BAD_PAGE and that key is skipped; a row naming a nonexistent request sets TV_STATUS_BAD_REQUEST.
  */
 typedef struct tv_tree_attention_fp32_args {
     /* q [Q, Hq, D], head dim contiguous */

@@ -30,13 +30,16 @@
 //     one product each: all 24 bits of it in bf16; in f16 to 2^-39 of the row's reference
 //     (Op<_Float16>), which is below what fp32 sums of it keep.
 //
+// Short requests take the row form (tv_attention_rows.hip; row_form_keys has the rule).
+//
 // What bounds it.  f32: the matrix core, 8192 cycles a tile and wave (a wave's tile takes 10.7 us
-// with two waves a SIMD, 7 us at the core's rate), and the uneven lengths of the workgroups.
+// with two waves a SIMD, 7 us at the core's rate), scratch traffic (16 to 66 spilled VGPRs at
+// head sizes 80 to 128), and the uneven lengths of the workgroups.
 // 16 bits: the loads and the softmax's vector work (3 us a tile) and the workgroup's fixed time
 // (lookups 3, Q and first tile 3, waves' merge 3, partial rows 2.5 us).  Measured, before (a wave
 // per packed row, fp32 vector products, K/V staged in LDS) -> now: 8 f32 requests of 310-3304
-// keys and 18-64 nodes, 32/8 heads x 128: 525 -> 151 us (5.9 GFLOP; 42 us at the f32 matrix
-// rate); 4 bf16 requests of 1204-1998 keys, 24/8 heads x 96, 16-token pages: 481 -> 37 us;
+// keys and 18-64 nodes, 32/8 heads x 128: 523 -> 142 us (5.9 GFLOP; 42 us at the f32 matrix
+// rate); 4 bf16 requests of 1204-1998 keys, 24/8 heads x 96, 16-token pages: 490 -> 34 us;
 // 2 x 1500-row bf16 chunks, 32/8 x 128: 7.1 -> 0.69 ms; head size 512, bf16: 7.2 -> 0.87 ms.
 #include <math.h>
 #include <stdint.h>
