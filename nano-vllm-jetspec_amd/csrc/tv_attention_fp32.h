@@ -41,7 +41,7 @@ struct Fp32Params {
     float scale;          // softmax scale in the form's score units
     int32_t splits;       // chunks a row block's keys may be cut into
     int32_t slots;        // workgroups the chip runs at a time
-    int32_t places;       // workgroups of a cut launch, each with room for its partial rows
+    int32_t places;       // workgroups of a launch by list (a cut one has room for their partial rows); 0: by number
     int32_t min_chunk;    // tiles of the shortest chunk a block is cut into
     int32_t kv_heads;
     int32_t vec;          // K/V rows take vector loads

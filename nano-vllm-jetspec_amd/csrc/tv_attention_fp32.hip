@@ -63,6 +63,7 @@ constexpr int kCutRequests = kWave; // requests of a batch that is cut at most (
 // Shortest chunk: a workgroup's fixed time (about 15 us: lookups, Q, the waves' merge, the partial
 // rows) against its tiles' (a wave's takes 11 us in f32, 3 us in 16 bits).
 constexpr int kMinChunk32 = 8, kMinChunk16 = 16;
+constexpr int kWholeKeys = 1 << 30;   // as the shortest chunk: nothing is cut
 constexpr int32_t kMaxRowKeys = 256;    // the most keys of a request the row form takes
 constexpr int64_t kRowRequests = 1024;  // ... and requests (every workgroup reads the lengths of a captured launch)
 // Scores and maxima are kept in units of two octaves (natural units * log2(e) / 2): the factor is
@@ -168,8 +169,8 @@ __device__ __forceinline__ int wave_max(int x) {   // of non-negative values
     return __builtin_amdgcn_readlane(x, kWave - 1);
 }
 
-// The cut of a batch whose keys are split (p.splits > 1, at most kCutRequests requests), the
-// same in every wave that computes it: chunks of at most `target` tiles (cut_target), so that
+// The cut of a batch launched by list (p.places > 0, at most kCutRequests requests), the same in
+// every wave that computes it: chunks of at most `target` tiles (cut_target), so that
 // the workgroups fill the chip once (p.slots of them run at a time: a part-filled second round
 // would double the launch), or as many times as the row blocks alone do.  Lane l holds request l.
 struct Cut {
@@ -778,7 +779,7 @@ tree_attention_fp32_kernel(const Fp32Params p) {
     // Index -> (block, chunk) and KV head, head fastest: with 8 KV heads the blocks and chunks of one
     // head share an XCD (workgroup i runs on XCD i % 8), and so its K/V in that L2.
     RowBlock b;
-    if (p.splits == 1) {
+    if (p.places == 0) {
         const int64_t unit = p.unit0 + blockIdx.x;
         const int64_t number = unit / p.kv_heads;
         const int r = __builtin_amdgcn_readfirstlane(request_of_group(p.cu, p.groups, p.num_requests, number));
@@ -888,13 +889,12 @@ bool own_instance(int32_t d) {
 // f32 x 64, 64 keys, 24 rows 8 / 16.  In 16 bits the instances of their own are ahead from a few
 // dozen keys on (x 96, three heads: always; x 80, one head, 64 keys, 24 rows 13 / 18), the shared
 // ones, with their padding and element loads, behind for longer (x 72, 192 keys, 64 rows 28 / 35).
-// Beyond one round of its workgroups (two a CU) the row form loses its lead unless the matrix
-// form's are about as many (48 requests of 8 nodes, four heads: 36 / 54; of 24 nodes 83 / 85).
+// Beyond one round of its workgroups (two a CU, four packed rows each) the row form loses its lead:
+// 48 requests of 2 nodes, four heads, 32 keys 15 / 19; of 8 nodes, 64 keys 36 / 32.
 int32_t row_form_keys(int64_t total_queries, int64_t num_requests, int64_t groups, int64_t kv_heads, int32_t in_dtype,
                       int32_t head_dim, bool vec) {
     if (groups > 4 || num_requests > kRowRequests) return 0;
-    const int64_t row_groups_4 = (total_queries / 4 + num_requests + 1) * kv_heads;
-    if (row_groups_4 > 2 * kCus && 2 * row_groups_4 > 3 * row_groups(total_queries, num_requests, groups) * kv_heads) return 0;
+    if ((total_queries / 4 + num_requests / 2) * kv_heads > 2 * kCus) return 0;
     const bool own = vec && own_instance(head_dim), f32 = in_dtype == TV_F32, few_heads = groups <= 2;
     const bool full = total_queries * groups >= 20 * num_requests;   // score rows of the average request
     if (!f32 && own) return few_heads ? (full ? (head_dim <= 128 ? 64 : 0) : 32) : 0;
@@ -928,7 +928,7 @@ void launch_for_dims(const Fp32Params& p, const dim3& grid, hipStream_t s) {
 // The head sizes models use are compiled in; the others share an instance per power of two.
 template <typename T>
 void launch_for_type(const Fp32Params& p, uint32_t units, hipStream_t s) {
-    const dim3 grid(p.splits == 1 ? units : static_cast<uint32_t>(p.places));
+    const dim3 grid(p.places == 0 ? units : static_cast<uint32_t>(p.places));
     const int d = p.head_dim;
     if (p.vec && d == 64) {
         launch_for_dims<T, 64, true>(p, grid, s);
@@ -1115,6 +1115,7 @@ extern "C" int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* a,
     p.status = a->status;
     p.kv_heads = a->num_kv_heads;
     p.splits = 1;
+    p.places = 0;
     p.ws_o = nullptr;
     p.ws_ml = nullptr;
     if (workspace && (max_keys == 0 || max_keys > min_chunk_tiles(a->in_dtype) * kTile)) {
@@ -1134,6 +1135,17 @@ extern "C" int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* a,
             p.ws_ml = static_cast<float2*>(workspace);
             p.ws_o = reinterpret_cast<float*>(p.ws_ml + places * kBlockRows);
         }
+    }
+    // Whole keys, but more numbers than the chip takes at once: the idle numbers between the requests'
+    // blocks (group_start) would alternate with live ones and leave places empty, so the blocks are
+    // listed as a cut batch's are (48 f32 requests of 8 nodes and 248 keys, 32/8 heads x 128: 92 us
+    // by number, 69 listed; up to one round the search costs a microsecond for nothing, and beyond
+    // 2048 numbers most are live: of 60 nodes at head size 64, 154 by number, 165 listed).
+    if (p.places == 0 && a->num_requests <= kCutRequests && units > chip_slots(a->head_dim) &&
+        units <= kCutRows / 2) {
+        p.places = static_cast<int32_t>(units);
+        p.slots = chip_slots(a->head_dim);
+        p.min_chunk = kWholeKeys;
     }
     const int64_t elem = a->in_dtype == TV_F32 ? 4 : 2;
     p.vec = vector_rows(a->k_pool, a->k_stride, elem, a->head_dim) &&

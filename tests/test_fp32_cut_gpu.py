@@ -35,6 +35,20 @@ def test_edges_of_the_cut(label, prefixes, counts, groups, dtype):
     assert read_and_clear_status(DEV) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("requests", [63, 64, 65])
+def test_whole_keys_of_more_blocks_than_the_chip_takes_at_once(requests, dtype):
+    """Short enough not to be cut, long enough for the matrix form: listed up to 64 requests, by
+    number above."""
+    q, k, v, meta, *_ = make_case([150 + i for i in range(requests)], [1 + i % 13 for i in range(requests)], kv_heads=8,
+                                  groups=4, head_dim=80, dtype=dtype, block=16, seed=requests)
+    out = packed_tree_attention(q, k, v, meta, 80 ** -0.5, 4, output_dtype=torch.float32)
+    torch.cuda.synchronize()
+    error, _ = errors(out, oracle_rows(q, k, v, meta, 80 ** -0.5, list(range(requests)), rows_per_request=2))
+    assert error <= BOUND
+    assert read_and_clear_status(DEV) == 0
+
+
 def test_a_request_without_nodes_among_live_metadata():
     """Its rows are left alone, the others' are right."""
     q, k, v, meta, *_ = make_case((700, 900, 1200), (9, 12, 30), head_dim=96, dtype=torch.float32, seed=4)
