@@ -1139,7 +1139,7 @@ extern "C" int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* a,
     // Whole keys, but more numbers than the chip takes at once: the idle numbers between the requests'
     // blocks (group_start) would alternate with live ones and leave places empty, so the blocks are
     // listed as a cut batch's are (48 f32 requests of 8 nodes and 248 keys, 32/8 heads x 128: 92 us
-    // by number, 69 listed; up to one round the search costs a microsecond for nothing, and beyond
+    // by number, 55 listed; up to one round the search costs a microsecond for nothing, and beyond
     // 2048 numbers most are live: of 60 nodes at head size 64, 154 by number, 165 listed).
     if (p.places == 0 && a->num_requests <= kCutRequests && units > chip_slots(a->head_dim) &&
         units <= kCutRows / 2) {
@@ -1153,7 +1153,7 @@ extern "C" int tv_tree_attention_fp32_keys(const tv_tree_attention_fp32_args* a,
     const int64_t per = 16 / elem;
     p.q_vec = aligned(a->q, 16) && a->q_stride_row % per == 0 && a->q_stride_head % per == 0 && a->head_dim % per == 0;
     // A batch whose lengths the host knows takes its form here; otherwise both are launched and
-    // the one that is not the batch's exits.
+    // the one that is not the batch's exits (4 to 5 us of empty launches for a short batch).
     hipStream_t s = as_stream(stream);
     const int32_t rows_keys = row_form_keys(a->total_queries, a->num_requests, p.groups, a->num_kv_heads, a->in_dtype,
                                             a->head_dim, p.vec);
