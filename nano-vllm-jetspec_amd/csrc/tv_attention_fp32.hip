@@ -38,7 +38,7 @@
 // 16 bits: the loads and the softmax's vector work (3 us a tile) and the workgroup's fixed time
 // (lookups 3, Q and first tile 3, waves' merge 3, partial rows 2.5 us).  Measured, before (a wave
 // per packed row, fp32 vector products, K/V staged in LDS) -> now: 8 f32 requests of 310-3304
-// keys and 18-64 nodes, 32/8 heads x 128: 523 -> 142 us (5.9 GFLOP; 42 us at the f32 matrix
+// keys and 18-64 nodes, 32/8 heads x 128: 525 -> 138 us (5.9 GFLOP; 42 us at the f32 matrix
 // rate); 4 bf16 requests of 1204-1998 keys, 24/8 heads x 96, 16-token pages: 490 -> 34 us;
 // 2 x 1500-row bf16 chunks, 32/8 x 128: 7.1 -> 0.69 ms; head size 512, bf16: 7.2 -> 0.87 ms.
 #include <math.h>
